@@ -3,8 +3,9 @@
 // attention, the short-conv mix, row RMSNorm and the device-side synthetic
 // weight generator.
 //
-//   gemm_nt_kernel      attn_matmul_tiled_kernel (layer.cu:9-141) and
-//                       lm_head_gemm_kernel (model.cu:42-116) as one MFMA GEMM,
+//   gemm kernels        attn_matmul_tiled_kernel (layer.cu:9-141) and
+//                       lm_head_gemm_kernel (model.cu:42-116) as one MFMA GEMM
+//                       (gemm_skinny_kernel for few rows, gemm_split_kernel),
 //                       with the decoder's residual add_kernel (layer.cu:1860-
 //                       1880 at 1912-1913) fused into its epilogue
 //   embed_kernel        embedding_lookup_kernel (model.cu:18-32)
@@ -19,8 +20,11 @@
 //                       token-major pass
 #include "lfm_internal.h"
 
+#include <algorithm>
+
 #include "gpu_common.h"
 #include "mfma_tile.h"
+#include "split_tile.h"
 
 namespace lfm {
 
@@ -31,14 +35,14 @@ using moe::kThreads;
 // Dense GEMM: C = A . B^T (+ R)
 // ---------------------------------------------------------------------------
 
-// Epilogue stores of the dense GEMM: plain 16-byte buffer stores (the output
-// is consumed by the next kernel, not by other blocks of this one).
+// Epilogue stores of the dense GEMM (the output is consumed by the next
+// kernel, not by other blocks of this one).
 struct PlainOut {
   __amdgpu_buffer_rsrc_t rsrc;
   __device__ PlainOut(float *base, uint32_t bytes)
       : rsrc(__builtin_amdgcn_make_buffer_rsrc(base, 0, (int)bytes, moe::kBufferRsrcWord3)) {}
-  __device__ void store(uint32_t off, f32x4 v) const {
-    __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, off, 0, 0);
+  __device__ void store1(uint32_t off, float v) const {
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rsrc, off, 0, 0);
   }
 };
 
@@ -51,12 +55,8 @@ struct ResidualOut {
   __device__ ResidualOut(float *base, uint32_t bytes, const float *r)
       : rsrc(__builtin_amdgcn_make_buffer_rsrc(base, 0, (int)bytes, moe::kBufferRsrcWord3)),
         res(r) {}
-  __device__ void store(uint32_t off, f32x4 v) const {
-    const f32x4 r = moe::ld4(res + off / 4);
-    f32x4 o;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) o[j] = r[j] + v[j];
-    __builtin_amdgcn_raw_buffer_store_b128(o, rsrc, off, 0, 0);
+  __device__ void store1(uint32_t off, float v) const {
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, res[off / 4] + v), rsrc, off, 0, 0);
   }
 };
 
@@ -69,19 +69,24 @@ struct GemmArgs {
 };
 
 constexpr int kGroupM = 8;  // M tiles walked together (their B tiles are shared)
+constexpr int kGemmCUs = 256;
 
-// One 128x128 (or 64x128) tile per block.  Tile order: the dispatcher sends
-// block b to XCD b % 8, so consecutive tile indices are given to the blocks
-// of one XCD (its L2 then holds the A and B slabs its blocks share), and
-// within that range tiles run in groups of kGroupM M-tiles column by column,
-// so the blocks running together share B tiles and A tiles.
+// One 128x128 (or 64x128) split-bf16 tile per block (split_tile.h).  Tile
+// order: the dispatcher sends block b to XCD b % 8, so consecutive tile indices
+// are given to the blocks of one XCD (its L2 then holds the A and B slabs its
+// blocks share), and within that range tiles run in groups of kGroupM M-tiles
+// column by column, so the blocks running together share B tiles and A tiles.
+// Bound by the matrix cores' power: at 32768 x 3072 x 2048 (128-row tiles)
+// 1864 us = 221 TFLOP/s, where the fp32 instruction's tile took 2819 us = 146
+// and bf16 MFMAs alone on random operands reach 300 / 6; the clock drops to
+// 1.7 GHz and the MFMAs are busy 69 % of it.
 template <int BM, bool RES>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
-void gemm_nt_kernel(GemmArgs g) {
-  using TL = moe::Tile<BM>;
+void gemm_split_kernel(GemmArgs g) {
+  using TL = moe::SplitTile<BM, 128>;
   extern __shared__ float lds[];
-  __shared__ int s_aoff[BM];
-  const int ntm = (g.M + BM - 1) / BM, ntn = g.N / TL::BN;
+  __shared__ int s_aoff[TL::BM];
+  const int ntm = (g.M + TL::BM - 1) / TL::BM, ntn = g.N / TL::BN;
   const int ntiles = ntm * ntn;
   int t = blockIdx.x;
   if (ntiles % 8 == 0) t = (t % 8) * (ntiles / 8) + t / 8;
@@ -89,19 +94,155 @@ void gemm_nt_kernel(GemmArgs g) {
   const int grp = t / per_group, first_m = grp * kGroupM;
   const int gsz = min(ntm - first_m, kGroupM);
   const int r = t - grp * per_group;
-  const int m0 = (first_m + r % gsz) * BM, n0 = (r / gsz) * TL::BN;
-  const int rows = min(BM, g.M - m0);
-  if (threadIdx.x < BM) s_aoff[threadIdx.x] = threadIdx.x < rows ? (m0 + threadIdx.x) * g.K : 0;
+  const int m0 = (first_m + r % gsz) * TL::BM, n0 = (r / gsz) * TL::BN;
+  const int rows = min(TL::BM, g.M - m0);
+  for (int i = threadIdx.x; i < TL::BM; i += kThreads) s_aoff[i] = i < rows ? (m0 + i) * g.K : 0;
   __syncthreads();
   const uint32_t abytes = (uint32_t)((size_t)g.M * g.K * sizeof(float));
   const uint32_t cbytes = (uint32_t)((size_t)g.M * g.N * sizeof(float));
   const float *brow0 = g.B + (size_t)n0 * g.K;
   if (RES)
-    moe::mfma_tile<TL, false, ResidualOut>(lds, g.A, abytes, s_aoff, rows, brow0, g.K,
-                                           ResidualOut(g.C, cbytes, g.R), m0, g.N, n0, nullptr);
+    moe::split_tile<TL, false, ResidualOut>(lds, g.A, abytes, s_aoff, rows, brow0, g.K,
+                                            ResidualOut(g.C, cbytes, g.R), m0, g.N, n0, nullptr);
   else
-    moe::mfma_tile<TL, false, PlainOut>(lds, g.A, abytes, s_aoff, rows, brow0, g.K,
-                                        PlainOut(g.C, cbytes), m0, g.N, n0, nullptr);
+    moe::split_tile<TL, false, PlainOut>(lds, g.A, abytes, s_aoff, rows, brow0, g.K,
+                                         PlainOut(g.C, cbytes), m0, g.N, n0, nullptr);
+}
+
+// Small M: a block of NW waves computes RM x RN blocks of 16x16, each wave all
+// of them over its own slice of K with v_mfma_f32_16x16x4_f32, NS - 1 pieces of
+// 32 k ahead in registers, and no barrier until the waves' sums meet in LDS.
+// Few rows leave few tiles, so a tile that one CU works through from end to end
+// takes as long as the whole product: splitting K over a block's waves keeps
+// many loads in flight and small tiles keep every CU busy.  Loads follow the
+// memory (8 lanes read the 128 bytes of a row's piece): the MFMA's operand
+// layout, whose neighbouring lanes hold different rows, loads one lane's 16
+// bytes per cycle (37 B/ns per CU measured, 4x below contiguous lanes).  The
+// pieces pass through a wave-private LDS buffer into the operand layout, 16-byte
+// chunk c of row r at c ^ (r % 8).  The products are in transposed form (B rows
+// as the first operand), so a lane's four results are consecutive columns.
+template <int RM, int RN, int NW, int NS_> struct SkinnyCfg {
+  static constexpr int BM = RM * 16, BN = RN * 16, PITCH = BN + 4, NS = NS_;
+  static constexpr int STAGE = (BM + BN) * 32;  // floats of a wave's LDS buffer
+  static constexpr int RED = BM * PITCH;        // floats of a wave's sums
+  static constexpr size_t LDS_BYTES = (size_t)NW * (STAGE > RED ? STAGE : RED) * sizeof(float);
+};
+
+template <int RM, int RN, int NW, int NS, bool RES>
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2)))
+void gemm_skinny_kernel(GemmArgs g) {
+  using CF = SkinnyCfg<RM, RN, NW, NS>;
+  extern __shared__ float lds[];
+  const int ntm = (g.M + CF::BM - 1) / CF::BM, ntiles = ntm * (g.N / CF::BN);
+  int t = blockIdx.x;
+  if (ntiles % 8 == 0) t = (t % 8) * (ntiles / 8) + t / 8;
+  const int m0 = (t % ntm) * CF::BM, n0 = (t / ntm) * CF::BN;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 15, lq = lane >> 4;
+  const int K = g.K;
+  const __amdgpu_buffer_rsrc_t ar = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float *>(g.A), 0, (int)((uint32_t)g.M * K * 4u), moe::kBufferRsrcWord3);
+  const __amdgpu_buffer_rsrc_t br = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float *>(g.B + (size_t)n0 * K), 0, (int)((uint32_t)CF::BN * K * 4u), moe::kBufferRsrcWord3);
+  // pieces past the end come through empty descriptors (zeros, no traffic), so
+  // every load is unconditional and the compiler's count of loads in flight
+  // stays exact
+  const __amdgpu_buffer_rsrc_t none =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(g.B), 0, 0, moe::kBufferRsrcWord3);
+  // lane l of a load: row l / 8 of 8, 16-byte chunk l % 8
+  const int ll = lane >> 3, lc = lane & 7;
+  uint32_t aoff[2 * RM], boff[2 * RN];
+#pragma unroll
+  for (int i = 0; i < 2 * RM; ++i) {
+    const int row = m0 + 8 * i + ll;
+    aoff[i] = row < g.M ? (uint32_t)(row * K + 4 * lc) * 4u : moe::kTileOOB;
+  }
+#pragma unroll
+  for (int i = 0; i < 2 * RN; ++i) boff[i] = (uint32_t)((8 * i + ll) * K + 4 * lc) * 4u;
+
+  // this wave's pieces: [p0, p1)
+  const int np = K / 32, per = (np + NW - 1) / NW;
+  const int p0 = min(wave * per, np), p1 = min(p0 + per, np);
+  f32x4 sa[NS][2 * RM], sb[NS][2 * RN];
+  auto load = [&](int p, int set) {
+    const bool in = p < p1;
+    const __amdgpu_buffer_rsrc_t arp = in ? ar : none, brp = in ? br : none;
+    const int ks = in ? p * 128 : 0;
+#pragma unroll
+    for (int i = 0; i < 2 * RN; ++i)
+      sb[set][i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(brp, boff[i], ks, 0));
+#pragma unroll
+    for (int i = 0; i < 2 * RM; ++i)
+      sa[set][i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(arp, aoff[i], ks, 0));
+  };
+  // the wave's buffer: B rows, then A rows, of 32 floats
+  float *stage = lds + (size_t)wave * CF::STAGE;
+  float *wr = stage + ll * 32 + (lc ^ ll) * 4;
+  const float *rd = stage + lr * 32;
+  const int rc[2] = {(lq ^ (lr & 7)) * 4, ((lq + 4) ^ (lr & 7)) * 4};
+  f32x4 acc[RM][RN];
+#pragma unroll
+  for (int i = 0; i < RM; ++i)
+#pragma unroll
+    for (int j = 0; j < RN; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int s = 0; s < NS - 1; ++s) {
+    load(p0 + s, s);
+    // in the loop's order: mixed, its first wait would be for all of them
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  for (int p = p0; p < p1; p += NS) {
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      load(p + s + NS - 1, (s + NS - 1) % NS);
+      __builtin_amdgcn_sched_barrier(0);
+      // a wave's LDS operations complete in order: no wait between the writes
+      // and the reads, and none before the next piece's writes
+#pragma unroll
+      for (int i = 0; i < 2 * RN; ++i) moe::st4(wr + i * 256, sb[s][i]);
+#pragma unroll
+      for (int i = 0; i < 2 * RM; ++i) moe::st4(wr + (RN * 2 + i) * 256, sa[s][i]);
+      __builtin_amdgcn_wave_barrier();
+      f32x4 af[RM][2], bf[RN][2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int j = 0; j < RN; ++j) bf[j][h] = moe::ld4(rd + j * 512 + rc[h]);
+#pragma unroll
+        for (int i = 0; i < RM; ++i) af[i][h] = moe::ld4(rd + (RN + i) * 512 + rc[h]);
+      }
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int i = 0; i < RM; ++i)
+#pragma unroll
+            for (int j = 0; j < RN; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[j][h][q], af[i][h][q], acc[i][j], 0, 0, 0);
+    }
+  }
+
+  __syncthreads();  // every wave is done with its buffer
+  // lane l of a block: row l % 16, columns 4 (l / 16) .. + 3
+#pragma unroll
+  for (int i = 0; i < RM; ++i)
+#pragma unroll
+    for (int j = 0; j < RN; ++j)
+      moe::st4(lds + (size_t)(wave * CF::BM + 16 * i + lr) * CF::PITCH + 16 * j + 4 * lq, acc[i][j]);
+  __syncthreads();
+  for (int f = tid; f < CF::BM * RN * 4; f += NW * 64) {
+    const int row = f / (RN * 4), c4 = (f % (RN * 4)) * 4;
+    if (m0 + row >= g.M) break;  // later rows too
+    f32x4 v = moe::ld4(lds + (size_t)row * CF::PITCH + c4);
+#pragma unroll
+    for (int w = 1; w < NW; ++w) v += moe::ld4(lds + (size_t)(w * CF::BM + row) * CF::PITCH + c4);
+    const size_t o = (size_t)(m0 + row) * g.N + n0 + c4;
+    if (RES) v = moe::ld4(g.R + o) + v;
+    moe::st4(g.C + o, v);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -468,25 +609,53 @@ __global__ __launch_bounds__(256) void fill_kernel(float *dst, size_t n, float v
 // Launchers
 // ---------------------------------------------------------------------------
 
-static hipError_t lds_attr(const void *fn, size_t bytes) {
-  if (bytes <= 65536) return hipSuccess;
-  return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-}
-
 template <int BM, bool RES>
-static hipError_t gemm_launch(const GemmArgs &g, hipStream_t st) {
-  using TL = moe::Tile<BM>;
-  const size_t lds = TL::LDS_FLOATS * sizeof(float);
-  const void *fn = reinterpret_cast<const void *>(&gemm_nt_kernel<BM, RES>);
-  const hipError_t e = lds_attr(fn, lds);
-  if (e != hipSuccess) return e;
-  const int tiles = ((g.M + BM - 1) / BM) * (g.N / TL::BN);
-  hipLaunchKernelGGL((gemm_nt_kernel<BM, RES>), dim3(tiles), dim3(kThreads), lds, st, g);
+static hipError_t gemm_split_launch(const GemmArgs &g, hipStream_t st) {
+  using TL = moe::SplitTile<BM, 128>;
+  static_assert(TL::LDS_BYTES <= 65536, "no LDS attribute needed");
+  const int tiles = ((g.M + TL::BM - 1) / TL::BM) * (g.N / TL::BN);
+  hipLaunchKernelGGL((gemm_split_kernel<BM, RES>), dim3(tiles), dim3(kThreads), TL::LDS_BYTES, st, g);
   return hipGetLastError();
 }
 
-// 64-row tiles for small M (the LM head's batch of last tokens), 128 above.
-constexpr int kGemmSmallM = 1024;
+template <int RM, int RN, int NW, int NS, bool RES>
+static hipError_t gemm_skinny_launch(const GemmArgs &g, hipStream_t st) {
+  using CF = SkinnyCfg<RM, RN, NW, NS>;
+  static_assert(CF::LDS_BYTES <= 65536, "no LDS attribute needed");
+  const int tiles = ((g.M + CF::BM - 1) / CF::BM) * (g.N / CF::BN);
+  hipLaunchKernelGGL((gemm_skinny_kernel<RM, RN, NW, NS, RES>), dim3(tiles), dim3(NW * 64), CF::LDS_BYTES, st, g);
+  return hipGetLastError();
+}
+
+template <bool RES>
+static hipError_t gemm_dispatch(const GemmArgs &g, hipStream_t st) {
+  // The kernel whose tiles are expected to take the least time over the CUs:
+  // blocks per CU, rounded up, times a block's share of a busy CU, at least the
+  // time of one block alone (us at K = 2048; every kernel's grows with K
+  // alike).  Measured against each other (us; tiles 16x16 / 16x32 / 32x32 with
+  // K split over waves, 64x128 / 128x128):
+  //   M=9    N=2048     6.1 /  8.6 /  13.4 /   71 /  105
+  //   M=9    N=6144    12.8 / 12.4 /  14.4 /   75 /  105
+  //   M=100  N=3072    23.3 / 19.5 /  21.4 /   71 /  105
+  //   M=154  N=6144    62   / 50   /  41   /   74 /  106
+  //   M=333  N=6144   109   / 90   /  80   /   89 /  107
+  //   M=64   N=65536  266   / 219  / 172   /  137 /  181
+  //   M=2664 N=2048     - / - / 309 /  142 /  147
+  //   M=2664 N=6144     - / - /  -  /  366 /  335
+  auto rounds = [&](long long bm, long long bn) {
+    return (double)(((g.M + bm - 1) / bm * (g.N / bn) + kGemmCUs - 1) / kGemmCUs);
+  };
+  const double cost[5] = {2.0 + 4.1 * rounds(16, 16), 1.5 + 6.2 * rounds(16, 32),
+                          4.0 + 9.0 * rounds(32, 32), std::max(71.0, 46.0 * rounds(64, 128)),
+                          std::max(103.0, 78.0 * rounds(128, 128))};
+  switch (std::min_element(cost, cost + 5) - cost) {
+    case 0: return gemm_skinny_launch<1, 1, 8, 4, RES>(g, st);
+    case 1: return gemm_skinny_launch<1, 2, 8, 4, RES>(g, st);
+    case 2: return gemm_skinny_launch<2, 2, 4, 4, RES>(g, st);
+    case 3: return gemm_split_launch<64, RES>(g, st);
+    default: return gemm_split_launch<128, RES>(g, st);
+  }
+}
 
 hipError_t launch_gemm_nt(const float *A, const float *B, float *C, const float *R, int M, int N,
                           int K, hipStream_t st) {
@@ -495,8 +664,7 @@ hipError_t launch_gemm_nt(const float *A, const float *B, float *C, const float 
   if ((size_t)M * K * sizeof(float) >= moe::kTileOOB || (size_t)M * N * sizeof(float) >= moe::kTileOOB)
     return hipErrorInvalidValue;
   const GemmArgs g{A, B, C, R, M, N, K};
-  if (M <= kGemmSmallM) return R ? gemm_launch<64, true>(g, st) : gemm_launch<64, false>(g, st);
-  return R ? gemm_launch<128, true>(g, st) : gemm_launch<128, false>(g, st);
+  return R ? gemm_dispatch<true>(g, st) : gemm_dispatch<false>(g, st);
 }
 
 hipError_t launch_embed(const int *ids, const float *table, float *h, int T, int H, int V, int *bad,

@@ -1,4 +1,4 @@
-// MFMA tile of the grouped and dense GEMMs: C = A . B^T on
+// MFMA tile of the grouped GEMM (32- and 64-row plans): C = A . B^T on
 // v_mfma_f32_32x32x2_f32, LDS double-buffered slabs with global loads three
 // slabs ahead.
 #pragma once

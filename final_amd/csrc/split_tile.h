@@ -1,0 +1,257 @@
+// Split-bf16 tile of the dense and grouped GEMMs: C = A . B^T for fp32 A and B
+// on v_mfma_f32_32x32x16_bf16.
+//
+// The fp32 matrix instruction peaks at 157 TFLOP/s on this chip, the bf16 one
+// at 2.5 PFLOP/s.  Every fp32 value is exactly the sum of three bf16 values
+// (8 significand bits each, rounded to nearest, so each part is at most 2^-9
+// of the one before), and a product of two values is then six bf16 products
+//   a2 b0 + a0 b2 + a1 b1 + a1 b0 + a0 b1 + a0 b0
+// plus three terms of at most 3 * 2^-27 of it, less than the rounding of one
+// fp32 product.  The six are exact in fp32 and accumulate in fp32, 16 k per
+// instruction, so a sum of K products takes 6 K / 16 roundings where the fp32
+// instruction takes K / 2: measured against 64-bit sums its error is smaller.
+// Six of them take 192 cycles per 32x32x16 block where fp32 takes 512.
+//
+// Values the split cannot carry (infinities, NaN, magnitudes above the largest
+// bf16, which round to infinity) leave a NaN or an infinity in every output
+// they reach, as does an fp32 overflow: a wave that finds one in its outputs
+// computes them again with the fp32 instruction.
+#pragma once
+
+#include "gpu_common.h"
+#include "mfma_tile.h"
+
+namespace moe {
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// x, y -> the packed bf16 pairs of their three parts (11 VALU operations).
+__device__ __forceinline__ void split_pair(float x, float y, uint32_t &p0, uint32_t &p1, uint32_t &p2) {
+  p0 = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{x, y}, bf16x2));
+  x -= __builtin_bit_cast(float, p0 << 16);
+  y -= __builtin_bit_cast(float, p0 & 0xFFFF0000u);
+  p1 = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{x, y}, bf16x2));
+  x -= __builtin_bit_cast(float, p1 << 16);
+  y -= __builtin_bit_cast(float, p1 & 0xFFFF0000u);
+  p2 = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{x, y}, bf16x2));
+}
+
+// Eight floats, as two float4s, to the three parts' operand registers.
+__device__ __forceinline__ void split8(const f32x4 (&v)[2], bf16x8 (&out)[3]) {
+  u32x4 p[3];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    uint32_t p0, p1, p2;
+    split_pair(v[j >> 1][(j & 1) * 2], v[j >> 1][(j & 1) * 2 + 1], p0, p1, p2);
+    p[0][j] = p0;
+    p[1][j] = p1;
+    p[2][j] = p2;
+  }
+#pragma unroll
+  for (int q = 0; q < 3; ++q) out[q] = __builtin_bit_cast(bf16x8, p[q]);
+}
+
+// The six products in ascending size, as (part of A, part of B).
+constexpr int kSplitProducts = 6;
+__device__ constexpr int kSplitA[kSplitProducts] = {2, 0, 1, 1, 0, 0};
+__device__ constexpr int kSplitB[kSplitProducts] = {0, 2, 1, 0, 1, 0};
+
+__device__ __forceinline__ bool not_finite(float v) {
+  return (__builtin_bit_cast(uint32_t, v) & 0x7F800000u) == 0x7F800000u;
+}
+
+// Tile of BM rows x BN columns, each of the four waves AM x 2 blocks of 32x32
+// (BN = 128: 2 x 2 waves, BN = 64: 4 x 1).  Slabs of 32 k: thread t stages 8
+// floats of rows t / 4 + 64 i (two float4s, 16 k apart, so four threads read
+// 64 contiguous bytes), splits them and writes one 16-byte chunk per plane;
+// both operands permute k alike.
+// Neighbouring lanes must hold neighbouring addresses: a load whose lanes hold
+// different rows moves 16 bytes per cycle, not 64.  LDS holds [3 planes][rows][4 chunks], chunk
+// c of row r at c ^ swizzle(r), so the 16-byte reads of neighbouring rows fall
+// in different banks without padding (no conflicts counted) and several blocks
+// share a CU: one splits its next slab while another's MFMAs run.
+template <int BM_, int BN_> struct SplitTile {
+  static constexpr int BM = BM_, BN = BN_, BK = 32;
+  static constexpr int WAVES_N = BN / 64, WAVES_M = kThreads / 64 / WAVES_N;
+  static constexpr int AM = BM / 32 / WAVES_M;  // 32-row blocks per wave
+  static constexpr int A_PASSES = BM / 64, PASSES = (BM + BN) / 64;  // float4 pairs per thread and slab
+  static constexpr int PLANE = (BM + BN) * BK;  // bf16 values per plane
+  static constexpr size_t LDS_BYTES = (size_t)3 * PLANE * 2;
+  static_assert(BM % 64 == 0 && (BN == 64 || BN == 128) && AM * WAVES_M * 32 == BM, "whole row blocks");
+};
+
+__device__ __forceinline__ int split_swizzle(int r) { return ((r >> 1) & 3) ^ ((r >> 3) & 1); }
+
+// Arguments as mfma_tile's (mfma_tile.h); out.store1(byte offset, value)
+// stores one float.  GATED: B rows come in groups of 32 of W1 and 32 of W3, a
+// wave's two column blocks, and silu(W1 x) * (W3 x) is stored.
+template <typename TL, bool GATED, typename Out, typename Ready = NoWait, typename Claim = int *>
+__device__ __forceinline__ int split_tile(float *lds, const float *abase, uint32_t abytes,
+                                          const int *aoff, int rows_valid, const float *brow0, int K,
+                                          const Out &out, int row0, int ldo, int col0, Claim head,
+                                          Ready ready = Ready{}) {
+  constexpr int AM = TL::AM, BM = TL::BM, PA = TL::A_PASSES, PASSES = TL::PASSES;
+  uint16_t *planes = reinterpret_cast<uint16_t *>(lds);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const __amdgpu_buffer_rsrc_t ar =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(abase), 0, (int)abytes, kBufferRsrcWord3);
+  const __amdgpu_buffer_rsrc_t br = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float *>(brow0), 0, (int)((uint32_t)TL::BN * K * 4u), kBufferRsrcWord3);
+
+  // staging: row lrow + 64 i (A rows, then B rows), float4s lq and lq + 4
+  const int lrow = tid >> 2, lq = tid & 3;
+  uint32_t a_src[PA];
+#pragma unroll
+  for (int i = 0; i < PA; ++i) {
+    const int r = lrow + 64 * i;
+    a_src[i] = r < rows_valid ? (uint32_t)(aoff[r] + lq * 4) * 4u : kTileOOB;
+  }
+  const uint32_t b_src = (uint32_t)(lrow * K + lq * 4) * 4u;
+  // slabs past the end come through empty descriptors: zeros, no traffic, and
+  // the compiler's count of loads in flight stays exact across the loop
+  const __amdgpu_buffer_rsrc_t none =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(brow0), 0, 0, kBufferRsrcWord3);
+  const int nslab = K / TL::BK;
+  f32x4 st[PASSES][2];
+  auto load = [&](int slab) {
+    const bool in = slab < nslab;
+    const __amdgpu_buffer_rsrc_t arp = in ? ar : none, brp = in ? br : none;
+    const int ks = in ? slab * TL::BK * 4 : 0;
+#pragma unroll
+    for (int i = 0; i < PASSES; ++i) {
+      const uint32_t off = i < PA ? a_src[i < PA ? i : 0] : b_src + (uint32_t)((i - PA) * 64 * K) * 4u;
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        st[i][h] = __builtin_bit_cast(
+            f32x4, __builtin_amdgcn_raw_buffer_load_b128(i < PA ? arp : brp, off + 64 * h, ks, 0));
+    }
+  };
+  // (lrow + 64 i) * 32 keeps lrow's swizzle: 64 i changes neither of its bits
+  uint16_t *wr = planes + lrow * TL::BK + (lq ^ split_swizzle(lrow)) * 8;
+  auto store = [&]() {
+#pragma unroll
+    for (int i = 0; i < PASSES; ++i) {
+      bf16x8 p[3];
+      split8(st[i], p);
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+        *reinterpret_cast<bf16x8 *>(wr + q * TL::PLANE + i * 64 * TL::BK) = p[q];
+    }
+  };
+
+  // fragments: lane l supplies row l % 32, chunk 2 kk + l / 32 of a slab
+  const int wm = wave % TL::WAVES_M, wn = wave / TL::WAVES_M;
+  const int lr = lane & 31, lh = lane >> 5;
+  const int sw = split_swizzle(lr);  // row blocks are 32 rows apart: the same swizzle
+  const uint16_t *a_rd = planes + (wm * AM * 32 + lr) * TL::BK;
+  const uint16_t *b_rd = planes + (BM + wn * 64 + lr) * TL::BK;
+  floatx16 acc[AM][2];
+#pragma unroll
+  for (int i = 0; i < AM; ++i)
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][c][r] = 0.0f;
+
+  if constexpr (Ready::kActive) {
+    if (wave == 0) ready.wait(0);
+    __syncthreads();
+  }
+  load(0);
+  for (int t = 0; t < nslab; ++t) {
+    store();
+    // the A columns of the slab loaded next, before the barrier
+    if constexpr (Ready::kActive)
+      if (wave == 0) ready.wait(t + 1);
+    __syncthreads();
+    // one slab ahead: two cost a block per CU in registers (64-row tiles,
+    // M=2664 N=K=2048: 141 us, 177 with two)
+    load(t + 1);
+    __builtin_amdgcn_sched_barrier(0);  // not sunk among the MFMAs
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      const int co = ((2 * kk + lh) ^ sw) * 8;
+      bf16x8 bf[2][3];
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int p = 0; p < 3; ++p)
+          bf[c][p] = *reinterpret_cast<const bf16x8 *>(b_rd + p * TL::PLANE + c * 32 * TL::BK + co);
+#pragma unroll
+      for (int i = 0; i < AM; ++i) {
+        bf16x8 af[3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p)
+          af[p] = *reinterpret_cast<const bf16x8 *>(a_rd + p * TL::PLANE + i * 32 * TL::BK + co);
+#pragma unroll
+        for (int m = 0; m < kSplitProducts; ++m)
+#pragma unroll
+          for (int c = 0; c < 2; ++c)
+            acc[i][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[kSplitA[m]], bf[c][kSplitB[m]],
+                                                                acc[i][c], 0, 0, 0);
+      }
+    }
+    __syncthreads();
+  }
+
+  const int next = tid == 0 ? claim_next(head) : 0;
+
+  // Results: lane l holds column l % 32 and rows 8 (r / 4) + 4 (l / 32) + r % 4
+  // of each block, so a store writes 128 contiguous bytes of two rows.
+  auto emit = [&](int i, const floatx16 &c0, const floatx16 &c1) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int row = wm * AM * 32 + i * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
+      if (row < rows_valid) {
+        const size_t o = (size_t)(row0 + row) * ldo + col0;
+        if (GATED) {
+          out.store1((uint32_t)((o + wn * 32 + lr) * 4), silu(c0[r]) * c1[r]);
+        } else {
+          out.store1((uint32_t)((o + wn * 64 + lr) * 4), c0[r]);
+          out.store1((uint32_t)((o + wn * 64 + 32 + lr) * 4), c1[r]);
+        }
+      }
+    }
+  };
+  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < AM; ++i)
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) bad |= not_finite(acc[i][c][r]);
+  if (!__any(bad)) {
+#pragma unroll
+    for (int i = 0; i < AM; ++i) emit(i, acc[i][0], acc[i][1]);
+  } else {
+    // fp32 MFMAs with operands straight from memory: lane l supplies row
+    // l % 32 at k offset 4 (l / 32) of each 8-wide k group
+    const uint32_t bo = (uint32_t)((wn * 64 + lr) * K + 4 * lh) * 4u;
+    for (int i = 0; i < AM; ++i) {
+      const int row = wm * AM * 32 + i * 32 + lr;
+      const uint32_t ao = row < rows_valid ? (uint32_t)(aoff[row] + 4 * lh) * 4u : kTileOOB;
+      floatx16 c[2];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) c[0][r] = c[1][r] = 0.0f;
+      for (int k = 0; k < K; k += 8) {
+        const f32x4 a = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ar, ao, k * 4, 0));
+        const f32x4 b0 = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(br, bo, k * 4, 0));
+        const f32x4 b1 = __builtin_bit_cast(
+            f32x4, __builtin_amdgcn_raw_buffer_load_b128(br, bo + (uint32_t)(32 * K) * 4u, k * 4, 0));
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          c[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q], b0[q], c[0], 0, 0, 0);
+          c[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q], b1[q], c[1], 0, 0, 0);
+        }
+      }
+      emit(i, c[0], c[1]);
+    }
+  }
+  return next;
+}
+
+}  // namespace moe

@@ -59,6 +59,67 @@ def test_gemm_nt(M, N, K, res, oracle_mod):
     np.testing.assert_allclose(got, ref, rtol=RTOL, atol=ATOL)
 
 
+# Sizes at the edges of every kernel of the GEMM's dispatch: 16x16, 16x32 and
+# 32x32 tiles with K split over waves, 64- and 128-row tiles; K of one slab,
+# of an odd number of slabs, and fewer pieces than waves.
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1, 128, 32), (16, 2048, 288), (17, 2048, 96), (112, 3072, 2048),
+                                   (113, 3072, 160), (97, 6144, 64), (333, 6144, 1056),
+                                   (65, 32768, 32), (64, 32768, 96), (1000, 6144, 2048),
+                                   (1009, 6144, 96), (2049, 6144, 32), (2049, 6144, 96),
+                                   (2720, 6144, 1792)])
+@pytest.mark.parametrize("res", [False, True])
+def test_gemm_nt_dispatch_edges(M, N, K, res):
+    from final_amd import hip, lfm
+    say(f"[gemm edges] M={M} N={N} K={K} residual={res}")
+    r = rng(M + N + K)
+    A = r.standard_normal((M, K), dtype=np.float32)
+    B = (0.02 * r.standard_normal((N, K), dtype=np.float32))
+    R = r.standard_normal((M, N), dtype=np.float32) if res else None
+    dA, dB = dev(A), dev(B)
+    dC = dev(R) if res else hip.DeviceArray((M, N))
+    lfm.gemm_nt(dA, dB, dC, M, N, K, R=dC if res else None)
+    got = dC.download()
+    cols = np.unique(r.integers(0, N, 300))  # a sample of the columns, in 64 bits
+    ref = A.astype(np.float64) @ B[cols].astype(np.float64).T
+    # K + 6 roundings of at most 2^-24 of the sum of the products' magnitudes
+    # (an fp32 sum in any order, whole or as bf16 parts), one more for the residual
+    tol = (K + 6) * 2.0 ** -24 * (np.abs(A).astype(np.float64) @ np.abs(B[cols]).astype(np.float64).T)
+    if res:
+        ref = R[:, cols] + ref
+        tol = tol + 2.0 ** -24 * np.abs(ref)
+    assert np.isfinite(got).all()
+    assert (np.abs(got[:, cols] - ref) <= tol).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N", [(40, 2048), (100, 3072), (65, 32768), (2049, 6144)])
+def test_gemm_nt_values_outside_bf16(M, N):
+    """Infinities, NaN and finite values above the largest bf16 give what fp32 arithmetic gives."""
+    from final_amd import hip, lfm
+    K = 96
+    r = rng(M)
+    A = r.standard_normal((M, K), dtype=np.float32)
+    B = (0.02 * r.standard_normal((N, K), dtype=np.float32))
+    big = np.float32(3.4e38)  # rounds to infinity in bf16
+    A[3, 5], A[9, 70], A[M - 1, 0] = np.inf, np.nan, -np.inf
+    A[20], A[20, 7] = 0.0, big  # products below overflow
+    B[N - 2], B[N - 2, 40] = 0.0, big
+    A[:, 40] = np.where(np.isfinite(A[:, 40]), 0.5, A[:, 40])
+    A[20, 40] = 0.0
+    dA, dB, dC = dev(A), dev(B), hip.DeviceArray((M, N))
+    lfm.gemm_nt(dA, dB, dC, M, N, K)
+    got = dC.download()
+    with np.errstate(all="ignore"):
+        ref = A.astype(np.float64) @ B.astype(np.float64).T
+        mag = np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64).T
+    fin = np.isfinite(ref)
+    assert not fin[[3, 9, M - 1]].all() and fin[20].all() and np.abs(ref[20]).max() > 1e37
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(got[~fin & ~np.isnan(ref)], ref[~fin & ~np.isnan(ref)])
+    assert (np.abs(got[fin] - ref[fin]) <= (K + 6) * 2.0 ** -24 * mag[fin]).all()
+
+
 @pytest.mark.gpu
 def test_embedding_bit_exact_and_bad_ids(oracle_mod):
     from final_amd import hip, lfm

@@ -75,6 +75,10 @@ struct AgentOut {
   __device__ void store(uint32_t byte_off, f32x4 v) const {
     __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, byte_off, 0, kCachePolicySc1);
   }
+  // one float per lane, where a wave's lanes write whole 128-byte lines
+  __device__ void store1(uint32_t byte_off, float v) const {
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rsrc, byte_off, 0, kCachePolicySc1);
+  }
 };
 
 // Block-wide: wait until *p >= target (thread 0 polls), then acquire.

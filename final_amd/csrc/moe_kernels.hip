@@ -34,6 +34,7 @@
 
 #include "gpu_common.h"
 #include "mfma_tile.h"
+#include "split_tile.h"
 
 namespace moe {
 
@@ -1820,17 +1821,17 @@ void expert_mfma_kernel(ExpertArgs a) {
         }
       } else if (BM == 128 && ghalf) {  // one W1/W3 row group: 32 intermediate columns
         static_assert(TileHalf<64>::BN == TileHalf<128>::BN, "a half tile's columns");
-        using TH = TileHalf<128>;
+        using TH = SplitTile<128, 64>;
         const float *hrow0 = a.w.w13 + ((size_t)e * 2 * I + (size_t)nt * TH::BN) * H;
+        next = split_tile<TH, true>(lds, a.x, xbytes, s_aoff, rows, hrow0, H, inter_out, slot0, I,
+                                    nt * (TH::BN / 2), next_task);
+      } else if (BM == 128) {
         if (rows <= 64)
-          next = mfma_tile<TileHalf<64>, true>(lds, a.x, xbytes, s_aoff, rows, hrow0, H, inter_out,
-                                               slot0, I, nt * (TH::BN / 2), next_task);
+          next = split_tile<SplitTile<64, 128>, true>(lds, a.x, xbytes, s_aoff, rows, brow0, H, inter_out,
+                                                      slot0, I, nt * (TL::BN / 2), next_task);
         else
-          next = mfma_tile<TH, true>(lds, a.x, xbytes, s_aoff, rows, hrow0, H, inter_out, slot0, I,
-                                     nt * (TH::BN / 2), next_task);
-      } else if (BM == 128 && rows <= 64) {
-        next = mfma_tile<Tile<64>, true>(lds, a.x, xbytes, s_aoff, rows, brow0, H, inter_out, slot0,
-                                         I, nt * (TL::BN / 2), next_task);
+          next = split_tile<SplitTile<128, 128>, true>(lds, a.x, xbytes, s_aoff, rows, brow0, H, inter_out,
+                                                       slot0, I, nt * (TL::BN / 2), next_task);
       } else {
         next = mfma_tile<Tile<BM>, true>(lds, a.x, xbytes, s_aoff, rows, brow0, H, inter_out, slot0,
                                          I, nt * (TL::BN / 2), next_task);
@@ -1906,15 +1907,23 @@ void expert_mfma_kernel(ExpertArgs a) {
       if (half) {
         using TH = TileHalf<BM>;
         const float *brow0 = a.w.w2 + ((size_t)e * H + (size_t)ht * TH::BN) * I;
-        next = mfma_tile<TH, false>(lds, abase, abytes, s_aoff, rows, brow0, I, sout_out, slot0,
-                                    H, ht * TH::BN, next_task, ready);
+        if constexpr (BM == 128)
+          next = split_tile<SplitTile<128, TH::BN>, false>(lds, abase, abytes, s_aoff, rows, brow0, I,
+                                                           sout_out, slot0, H, ht * TH::BN, next_task, ready);
+        else
+          next = mfma_tile<TH, false>(lds, abase, abytes, s_aoff, rows, brow0, I, sout_out, slot0,
+                                      H, ht * TH::BN, next_task, ready);
         tile_combine<TH::BN>(a, slot0, rows, ht * TH::BN, s_comb, &s_ncomb, row_tok, pmask);
       } else {
         const float *brow0 = a.w.w2 + ((size_t)e * H + (size_t)ht * TL::BN) * I;
-        if (BM == 128 && rows <= 64)
-          next = mfma_tile<Tile<64>, false>(lds, abase, abytes, s_aoff, rows, brow0, I, sout_out,
-                                            slot0, H, ht * TL::BN, next_task, ready);
-        else
+        if constexpr (BM == 128) {
+          if (rows <= 64)
+            next = split_tile<SplitTile<64, 128>, false>(lds, abase, abytes, s_aoff, rows, brow0, I, sout_out,
+                                                         slot0, H, ht * TL::BN, next_task, ready);
+          else
+            next = split_tile<SplitTile<128, 128>, false>(lds, abase, abytes, s_aoff, rows, brow0, I, sout_out,
+                                                          slot0, H, ht * TL::BN, next_task, ready);
+        } else
           next = mfma_tile<TL, false>(lds, abase, abytes, s_aoff, rows, brow0, I, sout_out, slot0,
                                       H, ht * TL::BN, next_task, ready);
         tile_combine<TL::BN>(a, slot0, rows, ht * TL::BN, s_comb, &s_ncomb, row_tok, pmask);
@@ -3282,7 +3291,7 @@ hipError_t launch_experts(const ExpertArgs &a, int tile_rows, int grid,
       break;
     }
     case 128: {
-      const size_t lds = Tile<128>::LDS_FLOATS * sizeof(float);
+      const size_t lds = SplitTile<128, 128>::LDS_BYTES;
       err = ensure_lds_attr(mfma_fn<128>(), lds);
       if (err != hipSuccess) return err;
       hipLaunchKernelGGL(expert_mfma_kernel<128>, dim3(grid), dim3(kThreads), lds, st, a);
@@ -3337,7 +3346,7 @@ int expert_blocks_per_cu(int tile_rows) {
       break;
     case 128:
       e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-          &n, mfma_fn<128>(), kThreads, Tile<128>::LDS_FLOATS * sizeof(float));
+          &n, mfma_fn<128>(), kThreads, SplitTile<128, 128>::LDS_BYTES);
       break;
     default:
       return 1;

@@ -185,22 +185,21 @@ static int plan_index(int rows) {
 // us at 8, 207.9 vs 211.5 at 9, 223.4 vs 225.1 at 10), 64-row MFMA tiles,
 // whose routing from score bounds planned in every block takes the router's
 // chains and planning off the critical path and whose down tiles all run at
-// half width up to 128 tokens, from 11 to 1024 tokens (231.1 vs 228.9 at
+// half width up to 128 tokens, from 11 to 560 tokens (231.1 vs 228.9 at
 // 11, 233.1 vs 230.2 at 12, 245.6 vs 235.1 at 16, 258.2 vs 243.5 at 20;
 // before the half-width down tiles streaming led up to 20; 283.3 vs 269.8
 // and 282.0 vs 276.3 at 48, two boxes;
-// equal at 640-768; 720 vs 726 at 832, 846 vs 854 at 1024), 128-row tiles
-// from 1025 (990 vs 1023 us at 1280, 1478 vs 1540 at 2048).  moe_route +
+// split-bf16 tiles from 321), 128-row tiles, all split-bf16, from 561 (495
+// vs 514 us at 512, 584 vs 530 at 640, 756 vs 685 at 1024).  moe_route +
 // moe_experts, which keep the full router, take the same plans (with it,
 // streaming led up to 48).
 constexpr int kStreamMaxTokens = 10;
-// The dense FFN's 4 chunk experts each hold every token, so its MFMA plans
-// have few tiles at small T: streaming stays fastest up to 192 tokens (214
-// vs 217 us at 128, 280 vs 283 at 192), 64-row tiles at 256 (290 vs 349 us),
-// 128-row tiles from 384 (433 vs 495 us at 512).
+// The dense FFN's 4 chunk experts each hold every token: streaming up to 192
+// tokens, 64-row split-bf16 tiles up to 640 (321 vs 372 us for 128-row tiles
+// at 512), 128-row tiles above (448 vs 420 at 768).
 static int auto_plan(int T, bool stream_ok, bool dense) {
   if (T <= (dense ? 192 : kStreamMaxTokens) && stream_ok) return 0;
-  if (T < (dense ? 384 : 1025)) return 64;
+  if (T < (dense ? 641 : 561)) return 64;
   return 128;
 }
 

@@ -30,6 +30,7 @@
 // order, so the smallest unfinished task is always running and every wait
 // ends; each wait is still bounded and reports MOE_ERR_DEVICE_TIMEOUT instead
 // of spinning forever.
+#include <algorithm>
 #include <type_traits>
 
 #include "gpu_common.h"
@@ -1626,8 +1627,17 @@ __device__ __forceinline__ int first_round_left(Ctrl *c, int f) {
   return -1;
 }
 
+// The 64-row plan's full-width tiles run as split-bf16 tiles (split_tile.h)
+// when its active experts hold more rows than this on average: below, the
+// units are padded and the 16-row fp32 layouts do less work (MoE block, whole
+// step, fp32 / split: 128 tokens 268 / 296 us, 256 306 / 328, 301 345 / 357,
+// 350 378 / 363, 400 417 / 387, 512 523 / 495).
+constexpr int kSplitMinRows = 40;
+using SplitUnit = SplitTile<64, 128, 2>;
+// 128-row plan: split-bf16 tiles only, three blocks per CU (three waves per
+// SIMD in 168 registers: 4096 tokens 2139 -> 1954 us, 16384 7808 -> 7122).
 template <int BM>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(BM == 128 ? 3 : 2)))
 void expert_mfma_kernel(ExpertArgs a) {
   using TL = Tile<BM>;
   extern __shared__ float lds[];
@@ -1635,7 +1645,7 @@ void expert_mfma_kernel(ExpertArgs a) {
   __shared__ int s_unit_off[kExperts + 1];
   __shared__ int s_full_off[kExperts + 1];  // unit order (unit_rows)
   __shared__ int s_pexp[kExperts];
-  __shared__ int s_nfull, s_lpt;
+  __shared__ int s_nfull, s_lpt, s_split;
   __shared__ int s_offsets[kExperts + 1];
   __shared__ int s_counts[kExperts];
   __shared__ int s_aoff[BM];
@@ -1697,7 +1707,9 @@ void expert_mfma_kernel(ExpertArgs a) {
     int nfull;
     s_full_off[tid] = lane_scan32(cnt / BM, tid, &nfull);
     const int npart = __popcll(__ballot(part > 0));
+    const int nactive = __popcll(__ballot(cnt > 0));
     if (tid == 0) {
+      s_split = !bounds && s_offsets[kExperts] > kSplitMinRows * nactive;
       s_full_off[kExperts] = nfull;
       s_nfull = nfull;
       s_lpt = 2 * nfull <= npart;
@@ -1716,6 +1728,7 @@ void expert_mfma_kernel(ExpertArgs a) {
   __syncthreads();
   const UnitOrder uo{s_unit_off, s_full_off, s_pexp, s_counts, BM <= 64 ? s_nfull : 0,
                      BM <= 64 && s_lpt != 0};
+  const bool split = BM == 64 && s_split != 0;
   // slots written by the router: gate/up tiles need not wait for the dispatch
   // tasks, which then only clear the combine counters (down tiles wait for
   // them) and write the rows of tokens without an expert
@@ -1815,6 +1828,9 @@ void expert_mfma_kernel(ExpertArgs a) {
           const float *hrow0 = a.w.w13 + ((size_t)e * 2 * I + (size_t)nt * TH::BN) * H;
           next = mfma_tile<TH, true>(lds, a.x, xbytes, s_aoff, rows, hrow0, H, inter_out, slot0,
                                      I, nt * (TH::BN / 2), next_task);
+        } else if (split) {
+          next = split_tile<SplitUnit, true>(lds, a.x, xbytes, s_aoff, rows, brow0, H, inter_out, slot0,
+                                            I, nt * (TL::BN / 2), next_task);
         } else {
           next = mfma_tile<TL, true>(lds, a.x, xbytes, s_aoff, rows, brow0, H, inter_out, slot0,
                                      I, nt * (TL::BN / 2), next_task);
@@ -1923,9 +1939,13 @@ void expert_mfma_kernel(ExpertArgs a) {
           else
             next = split_tile<SplitTile<128, 128>, false>(lds, abase, abytes, s_aoff, rows, brow0, I, sout_out,
                                                           slot0, H, ht * TL::BN, next_task, ready);
-        } else
+        } else if (split) {
+          next = split_tile<SplitUnit, false>(lds, abase, abytes, s_aoff, rows, brow0, I, sout_out, slot0,
+                                             H, ht * TL::BN, next_task, ready);
+        } else {
           next = mfma_tile<TL, false>(lds, abase, abytes, s_aoff, rows, brow0, I, sout_out, slot0,
                                       H, ht * TL::BN, next_task, ready);
+        }
         tile_combine<TL::BN>(a, slot0, rows, ht * TL::BN, s_comb, &s_ncomb, row_tok, pmask);
       }
     }
@@ -3251,6 +3271,8 @@ bool stream_supported(int H, int I) { return stream_fn(H, I) != nullptr; }
 
 int stream_max_tokens() { return kRingMaxSlots / kTopK; }
 
+// the 64-row plan's tiles, fp32 or split
+constexpr size_t kLds64 = std::max(Tile<64>::LDS_FLOATS * sizeof(float), SplitUnit::LDS_BYTES);
 template <int BM> static void *mfma_fn() {
   return reinterpret_cast<void *>(&expert_mfma_kernel<BM>);
 }
@@ -3284,7 +3306,7 @@ hipError_t launch_experts(const ExpertArgs &a, int tile_rows, int grid,
       break;
     }
     case 64: {
-      const size_t lds = Tile<64>::LDS_FLOATS * sizeof(float);
+      const size_t lds = kLds64;
       err = ensure_lds_attr(mfma_fn<64>(), lds);
       if (err != hipSuccess) return err;
       hipLaunchKernelGGL(expert_mfma_kernel<64>, dim3(grid), dim3(kThreads), lds, st, a);
@@ -3342,7 +3364,7 @@ int expert_blocks_per_cu(int tile_rows) {
       break;
     case 64:
       e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-          &n, mfma_fn<64>(), kThreads, Tile<64>::LDS_FLOATS * sizeof(float));
+          &n, mfma_fn<64>(), kThreads, kLds64);
       break;
     case 128:
       e = hipOccupancyMaxActiveBlocksPerMultiprocessor(

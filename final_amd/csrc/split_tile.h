@@ -28,7 +28,8 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// x, y -> the packed bf16 pairs of their three parts (11 VALU operations).
+// x, y -> the packed bf16 pairs of their three parts (11 VALU operations; with
+// integer rounding and byte permutes instead of conversions as fast).
 __device__ __forceinline__ void split_pair(float x, float y, uint32_t &p0, uint32_t &p1, uint32_t &p2) {
   p0 = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{x, y}, bf16x2));
   x -= __builtin_bit_cast(float, p0 << 16);
@@ -73,13 +74,20 @@ __device__ __forceinline__ bool not_finite(float v) {
 // c of row r at c ^ swizzle(r), so the 16-byte reads of neighbouring rows fall
 // in different banks without padding (no conflicts counted) and several blocks
 // share a CU: one splits its next slab while another's MFMAs run.
-template <int BM_, int BN_> struct SplitTile {
+template <int BM_, int BN_, int NBUF_ = 1> struct SplitTile {
   static constexpr int BM = BM_, BN = BN_, BK = 32;
+  // LDS slab buffers and slabs of global loads in flight.  One: two barriers
+  // per slab, the other blocks of the CU fill the waits (three blocks at 128
+  // rows).  Two: the next slab is split between the MFMAs of this one, one
+  // barrier per slab; faster where only two blocks fit anyway (64-row expert
+  // units, 512 tokens: 522 -> 495 us), slower where it costs a block (64-row
+  // dense tiles at M=2664 N=2048: 140 -> 155 us).
+  static constexpr int NBUF = NBUF_, NS = NBUF;
   static constexpr int WAVES_N = BN / 64, WAVES_M = kThreads / 64 / WAVES_N;
   static constexpr int AM = BM / 32 / WAVES_M;  // 32-row blocks per wave
   static constexpr int A_PASSES = BM / 64, PASSES = (BM + BN) / 64;  // float4 pairs per thread and slab
   static constexpr int PLANE = (BM + BN) * BK;  // bf16 values per plane
-  static constexpr size_t LDS_BYTES = (size_t)3 * PLANE * 2;
+  static constexpr size_t LDS_BYTES = (size_t)3 * PLANE * 2 * NBUF;
   static_assert(BM % 64 == 0 && (BN == 64 || BN == 128) && AM * WAVES_M * 32 == BM, "whole row blocks");
 };
 
@@ -116,8 +124,9 @@ __device__ __forceinline__ int split_tile(float *lds, const float *abase, uint32
   const __amdgpu_buffer_rsrc_t none =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(brow0), 0, 0, kBufferRsrcWord3);
   const int nslab = K / TL::BK;
-  f32x4 st[PASSES][2];
-  auto load = [&](int slab) {
+  constexpr int NS = TL::NS;
+  f32x4 st[NS][PASSES][2];
+  auto load = [&](int slab, int set) {
     const bool in = slab < nslab;
     const __amdgpu_buffer_rsrc_t arp = in ? ar : none, brp = in ? br : none;
     const int ks = in ? slab * TL::BK * 4 : 0;
@@ -126,20 +135,20 @@ __device__ __forceinline__ int split_tile(float *lds, const float *abase, uint32
       const uint32_t off = i < PA ? a_src[i < PA ? i : 0] : b_src + (uint32_t)((i - PA) * 64 * K) * 4u;
 #pragma unroll
       for (int h = 0; h < 2; ++h)
-        st[i][h] = __builtin_bit_cast(
+        st[set][i][h] = __builtin_bit_cast(
             f32x4, __builtin_amdgcn_raw_buffer_load_b128(i < PA ? arp : brp, off + 64 * h, ks, 0));
     }
   };
   // (lrow + 64 i) * 32 keeps lrow's swizzle: 64 i changes neither of its bits
   uint16_t *wr = planes + lrow * TL::BK + (lq ^ split_swizzle(lrow)) * 8;
-  auto store = [&]() {
+  auto store = [&](int set, int buf) {
 #pragma unroll
     for (int i = 0; i < PASSES; ++i) {
       bf16x8 p[3];
-      split8(st[i], p);
+      split8(st[set][i], p);
 #pragma unroll
       for (int q = 0; q < 3; ++q)
-        *reinterpret_cast<bf16x8 *>(wr + q * TL::PLANE + i * 64 * TL::BK) = p[q];
+        *reinterpret_cast<bf16x8 *>(wr + (3 * buf + q) * TL::PLANE + i * 64 * TL::BK) = p[q];
     }
   };
 
@@ -158,44 +167,70 @@ __device__ __forceinline__ int split_tile(float *lds, const float *abase, uint32
       for (int r = 0; r < 16; ++r) acc[i][c][r] = 0.0f;
 
   if constexpr (Ready::kActive) {
-    if (wave == 0) ready.wait(0);
+    if (wave == 0)
+      for (int j = 0; j < NS; ++j) ready.wait(j);
     __syncthreads();
   }
-  load(0);
-  for (int t = 0; t < nslab; ++t) {
-    store();
-    // the A columns of the slab loaded next, before the barrier
+#pragma unroll
+  for (int j = 0; j < NS; ++j) {
+    load(j, j);
+    __builtin_amdgcn_sched_barrier(0);  // in the loop's order: see the waits in it
+  }
+  auto compute = [&](int kk, int buf) {
+    const int co = ((2 * kk + lh) ^ sw) * 8 + 3 * buf * TL::PLANE;
+    bf16x8 bf[2][3];
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+        bf[c][p] = *reinterpret_cast<const bf16x8 *>(b_rd + p * TL::PLANE + c * 32 * TL::BK + co);
+#pragma unroll
+    for (int i = 0; i < AM; ++i) {
+      bf16x8 af[3];
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+        af[p] = *reinterpret_cast<const bf16x8 *>(a_rd + p * TL::PLANE + i * 32 * TL::BK + co);
+#pragma unroll
+      for (int m = 0; m < kSplitProducts; ++m)
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+          acc[i][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[kSplitA[m]], bf[c][kSplitB[m]],
+                                                              acc[i][c], 0, 0, 0);
+    }
+  };
+  if constexpr (TL::NBUF == 1) {
+    for (int t = 0; t < nslab; ++t) {
+      store(0, 0);
+      // the A columns of the slab loaded next, before the barrier
+      if constexpr (Ready::kActive)
+        if (wave == 0) ready.wait(t + 1);
+      __syncthreads();
+      load(t + 1, 0);
+      __builtin_amdgcn_sched_barrier(0);  // not sunk among the MFMAs
+      compute(0, 0);
+      compute(1, 0);
+      __syncthreads();
+    }
+  } else {
+    store(0, 0);
     if constexpr (Ready::kActive)
-      if (wave == 0) ready.wait(t + 1);
+      if (wave == 0) ready.wait(2);
     __syncthreads();
-    // one slab ahead: two cost a block per CU in registers (64-row tiles,
-    // M=2664 N=K=2048: 141 us, 177 with two)
-    load(t + 1);
-    __builtin_amdgcn_sched_barrier(0);  // not sunk among the MFMAs
+    for (int s = 0; s < nslab; s += 2) {
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      const int co = ((2 * kk + lh) ^ sw) * 8;
-      bf16x8 bf[2][3];
-#pragma unroll
-      for (int c = 0; c < 2; ++c)
-#pragma unroll
-        for (int p = 0; p < 3; ++p)
-          bf[c][p] = *reinterpret_cast<const bf16x8 *>(b_rd + p * TL::PLANE + c * 32 * TL::BK + co);
-#pragma unroll
-      for (int i = 0; i < AM; ++i) {
-        bf16x8 af[3];
-#pragma unroll
-        for (int p = 0; p < 3; ++p)
-          af[p] = *reinterpret_cast<const bf16x8 *>(a_rd + p * TL::PLANE + i * 32 * TL::BK + co);
-#pragma unroll
-        for (int m = 0; m < kSplitProducts; ++m)
-#pragma unroll
-          for (int c = 0; c < 2; ++c)
-            acc[i][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[kSplitA[m]], bf[c][kSplitB[m]],
-                                                                acc[i][c], 0, 0, 0);
+      for (int u = 0; u < 2; ++u) {
+        const int t = s + u;
+        if (t >= nslab) break;
+        load(t + 2, u);
+        __builtin_amdgcn_sched_barrier(0);
+        compute(0, u);
+        store(1 - u, 1 - u);  // slab t + 1 (past the end: zeros into a buffer nobody reads)
+        compute(1, u);
+        if constexpr (Ready::kActive)
+          if (wave == 0) ready.wait(t + 3);
+        __syncthreads();
       }
     }
-    __syncthreads();
   }
 
   const int next = tid == 0 ? claim_next(head) : 0;

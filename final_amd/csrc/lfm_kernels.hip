@@ -23,7 +23,7 @@
 #include <algorithm>
 
 #include "gpu_common.h"
-#include "mfma_tile.h"
+#include "skinny_tile.h"
 #include "split_tile.h"
 
 namespace lfm {
@@ -109,136 +109,27 @@ void gemm_split_kernel(GemmArgs g) {
                                          PlainOut(g.C, cbytes), m0, g.N, n0, nullptr);
 }
 
-// Small M: a block of NW waves computes RM x RN blocks of 16x16, each wave all
-// of them over its own slice of K with v_mfma_f32_16x16x4_f32, NS - 1 pieces of
-// 32 k ahead in registers, and no barrier until the waves' sums meet in LDS.
-// Few rows leave few tiles, so a tile that one CU works through from end to end
-// takes as long as the whole product: splitting K over a block's waves keeps
-// many loads in flight and small tiles keep every CU busy.  Loads follow the
-// memory (8 lanes read the 128 bytes of a row's piece): the MFMA's operand
-// layout, whose neighbouring lanes hold different rows, loads one lane's 16
-// bytes per cycle (37 B/ns per CU measured, 4x below contiguous lanes).  The
-// pieces pass through a wave-private LDS buffer into the operand layout, 16-byte
-// chunk c of row r at c ^ (r % 8).  The products are in transposed form (B rows
-// as the first operand), so a lane's four results are consecutive columns.
-template <int RM, int RN, int NW, int NS_> struct SkinnyCfg {
-  static constexpr int BM = RM * 16, BN = RN * 16, PITCH = BN + 4, NS = NS_;
-  static constexpr int STAGE = (BM + BN) * 32;  // floats of a wave's LDS buffer
-  static constexpr int RED = BM * PITCH;        // floats of a wave's sums
-  static constexpr size_t LDS_BYTES = (size_t)NW * (STAGE > RED ? STAGE : RED) * sizeof(float);
-};
-
-template <int RM, int RN, int NW, int NS, bool RES>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2)))
+// Few rows: one K-split tile per block (skinny_tile.h), the M tiles of a column
+// next to each other.
+template <typename CF, bool RES>
+__global__ __launch_bounds__(CF::NW * 64) __attribute__((amdgpu_waves_per_eu(2)))
 void gemm_skinny_kernel(GemmArgs g) {
-  using CF = SkinnyCfg<RM, RN, NW, NS>;
   extern __shared__ float lds[];
   const int ntm = (g.M + CF::BM - 1) / CF::BM, ntiles = ntm * (g.N / CF::BN);
   int t = blockIdx.x;
   if (ntiles % 8 == 0) t = (t % 8) * (ntiles / 8) + t / 8;
   const int m0 = (t % ntm) * CF::BM, n0 = (t / ntm) * CF::BN;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lr = lane & 15, lq = lane >> 4;
-  const int K = g.K;
-  const __amdgpu_buffer_rsrc_t ar = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<float *>(g.A), 0, (int)((uint32_t)g.M * K * 4u), moe::kBufferRsrcWord3);
-  const __amdgpu_buffer_rsrc_t br = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<float *>(g.B + (size_t)n0 * K), 0, (int)((uint32_t)CF::BN * K * 4u), moe::kBufferRsrcWord3);
-  // pieces past the end come through empty descriptors (zeros, no traffic), so
-  // every load is unconditional and the compiler's count of loads in flight
-  // stays exact
-  const __amdgpu_buffer_rsrc_t none =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(g.B), 0, 0, moe::kBufferRsrcWord3);
-  // lane l of a load: row l / 8 of 8, 16-byte chunk l % 8
-  const int ll = lane >> 3, lc = lane & 7;
-  uint32_t aoff[2 * RM], boff[2 * RN];
-#pragma unroll
-  for (int i = 0; i < 2 * RM; ++i) {
-    const int row = m0 + 8 * i + ll;
-    aoff[i] = row < g.M ? (uint32_t)(row * K + 4 * lc) * 4u : moe::kTileOOB;
-  }
-#pragma unroll
-  for (int i = 0; i < 2 * RN; ++i) boff[i] = (uint32_t)((8 * i + ll) * K + 4 * lc) * 4u;
-
-  // this wave's pieces: [p0, p1)
-  const int np = K / 32, per = (np + NW - 1) / NW;
-  const int p0 = min(wave * per, np), p1 = min(p0 + per, np);
-  f32x4 sa[NS][2 * RM], sb[NS][2 * RN];
-  auto load = [&](int p, int set) {
-    const bool in = p < p1;
-    const __amdgpu_buffer_rsrc_t arp = in ? ar : none, brp = in ? br : none;
-    const int ks = in ? p * 128 : 0;
-#pragma unroll
-    for (int i = 0; i < 2 * RN; ++i)
-      sb[set][i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(brp, boff[i], ks, 0));
-#pragma unroll
-    for (int i = 0; i < 2 * RM; ++i)
-      sa[set][i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(arp, aoff[i], ks, 0));
-  };
-  // the wave's buffer: B rows, then A rows, of 32 floats
-  float *stage = lds + (size_t)wave * CF::STAGE;
-  float *wr = stage + ll * 32 + (lc ^ ll) * 4;
-  const float *rd = stage + lr * 32;
-  const int rc[2] = {(lq ^ (lr & 7)) * 4, ((lq + 4) ^ (lr & 7)) * 4};
-  f32x4 acc[RM][RN];
-#pragma unroll
-  for (int i = 0; i < RM; ++i)
-#pragma unroll
-    for (int j = 0; j < RN; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-  for (int s = 0; s < NS - 1; ++s) {
-    load(p0 + s, s);
-    // in the loop's order: mixed, its first wait would be for all of them
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  for (int p = p0; p < p1; p += NS) {
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      load(p + s + NS - 1, (s + NS - 1) % NS);
-      __builtin_amdgcn_sched_barrier(0);
-      // a wave's LDS operations complete in order: no wait between the writes
-      // and the reads, and none before the next piece's writes
-#pragma unroll
-      for (int i = 0; i < 2 * RN; ++i) moe::st4(wr + i * 256, sb[s][i]);
-#pragma unroll
-      for (int i = 0; i < 2 * RM; ++i) moe::st4(wr + (RN * 2 + i) * 256, sa[s][i]);
-      __builtin_amdgcn_wave_barrier();
-      f32x4 af[RM][2], bf[RN][2];
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-#pragma unroll
-        for (int j = 0; j < RN; ++j) bf[j][h] = moe::ld4(rd + j * 512 + rc[h]);
-#pragma unroll
-        for (int i = 0; i < RM; ++i) af[i][h] = moe::ld4(rd + (RN + i) * 512 + rc[h]);
-      }
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-          for (int i = 0; i < RM; ++i)
-#pragma unroll
-            for (int j = 0; j < RN; ++j)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[j][h][q], af[i][h][q], acc[i][j], 0, 0, 0);
-    }
-  }
-
-  __syncthreads();  // every wave is done with its buffer
-  // lane l of a block: row l % 16, columns 4 (l / 16) .. + 3
-#pragma unroll
-  for (int i = 0; i < RM; ++i)
-#pragma unroll
-    for (int j = 0; j < RN; ++j)
-      moe::st4(lds + (size_t)(wave * CF::BM + 16 * i + lr) * CF::PITCH + 16 * j + 4 * lq, acc[i][j]);
-  __syncthreads();
-  for (int f = tid; f < CF::BM * RN * 4; f += NW * 64) {
-    const int row = f / (RN * 4), c4 = (f % (RN * 4)) * 4;
+  const float *b0 = g.B + (size_t)n0 * g.K;
+  moe::skinny_tile<CF>(
+      lds, g.A, g.M, m0, g.K / 32, (uint32_t)CF::BN * g.K * 4u, [&](int r) { return r * g.K; },
+      [&](int p, int &k0) {
+        k0 = p * 32;
+        return b0;
+      });
+  for (int f = threadIdx.x; f < CF::BM * CF::RN * 4; f += CF::NW * 64) {
+    const int row = f / (CF::RN * 4), c4 = (f % (CF::RN * 4)) * 4;
     if (m0 + row >= g.M) break;  // later rows too
-    f32x4 v = moe::ld4(lds + (size_t)row * CF::PITCH + c4);
-#pragma unroll
-    for (int w = 1; w < NW; ++w) v += moe::ld4(lds + (size_t)(w * CF::BM + row) * CF::PITCH + c4);
+    f32x4 v = moe::skinny_sum<CF>(lds, row, c4);
     const size_t o = (size_t)(m0 + row) * g.N + n0 + c4;
     if (RES) v = moe::ld4(g.R + o) + v;
     moe::st4(g.C + o, v);
@@ -620,10 +511,9 @@ static hipError_t gemm_split_launch(const GemmArgs &g, hipStream_t st) {
 
 template <int RM, int RN, int NW, int NS, bool RES>
 static hipError_t gemm_skinny_launch(const GemmArgs &g, hipStream_t st) {
-  using CF = SkinnyCfg<RM, RN, NW, NS>;
-  static_assert(CF::LDS_BYTES <= 65536, "no LDS attribute needed");
+  using CF = moe::SkinnyTile<RM, RN, NW, NS>;
   const int tiles = ((g.M + CF::BM - 1) / CF::BM) * (g.N / CF::BN);
-  hipLaunchKernelGGL((gemm_skinny_kernel<RM, RN, NW, NS, RES>), dim3(tiles), dim3(NW * 64), CF::LDS_BYTES, st, g);
+  hipLaunchKernelGGL((gemm_skinny_kernel<CF, RES>), dim3(tiles), dim3(NW * 64), CF::LDS_BYTES, st, g);
   return hipGetLastError();
 }
 

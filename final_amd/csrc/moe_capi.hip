@@ -758,6 +758,26 @@ int moe_dense_forward(moe_ctx *ctx, const float *x, float *y, const float *resid
   if (!x || !aligned16(x)) return MOE_ERR_INVALID_ARG;
   DeviceGuard g(ctx->device);
   if (!g.ok) return MOE_ERR_HIP;
+  if (ctx_plan(ctx, num_tokens) == 0 && dense_skinny_supported(ctx->d.hidden, ctx->dense_inter) &&
+      experts_args_ok(x, y, residual)) {
+    // the chunks' inter rows [4T][I / 4] hold the [T][I] of this path
+    DenseArgs da{};
+    da.x = x;
+    da.y = y;
+    da.residual = residual;
+    da.w13 = ctx->w13;
+    da.w2 = ctx->w2;
+    da.s = ctx->s;
+    da.T = num_tokens;
+    da.H = ctx->d.hidden;
+    da.I = ctx->dense_inter;
+    if (launch_dense_skinny(da, static_cast<hipStream_t>(stream)) != hipSuccess) return MOE_ERR_HIP;
+    ctx->routed_T = num_tokens;
+    ctx->route_pending = false;
+    ctx->routed_plan = 0;
+    ctx->routed_bounds = false;
+    return MOE_OK;
+  }
   RouterArgs a{};
   a.x = x;
   a.w.w13 = ctx->w13;

@@ -206,6 +206,19 @@ hipError_t launch_rmsnorm(const float *h, const float *w, float *out, int T, int
 // Fixed routing of the dense FFN (every token to chunks 0..kDenseChunks-1,
 // weight 1) and the plan for it; a.tile_rows/bn/inter as for launch_router.
 hipError_t launch_router_dense(const RouterArgs &a, hipStream_t st);
+// Dense FFN of few tokens as two K-split GEMMs (gate/up, down), in place of the
+// fixed routing and the streaming kernel.  y may alias the residual.
+struct DenseArgs {
+  const float *x;         // [T][H]
+  float *y;               // [T][H]
+  const float *residual;  // [T][H] or null
+  const float *w13;       // [I/32][2][32][H]
+  const float *w2;        // [kDenseChunks][H][I / kDenseChunks]
+  Scratch s;              // inter as [T][I]; idx, wts and the plan's counts get the fixed routing
+  int T, H, I;
+};
+hipError_t launch_dense_skinny(const DenseArgs &a, hipStream_t st);
+bool dense_skinny_supported(int H, int I);
 // Whether the weight-streaming kernel is compiled for (H, I).
 bool stream_supported(int H, int I);
 // Largest batch the streaming plan handles (its slot -> token map is in LDS).

@@ -35,6 +35,7 @@
 
 #include "gpu_common.h"
 #include "mfma_tile.h"
+#include "skinny_tile.h"
 #include "split_tile.h"
 
 namespace moe {
@@ -3155,6 +3156,81 @@ __global__ __launch_bounds__(kRingThreads) void expert_ring_kernel(ExpertArgs a)
 #define MOE_STREAM_SHAPES(X) X(8, 7)
 
 // ---------------------------------------------------------------------------
+// Dense FFN of few tokens: two K-split GEMMs (skinny_tile.h) on the chunked
+// weights.  The streaming kernel runs every token group's MFMAs behind one
+// task queue and its down rows behind the whole gate/up phase of a chunk; two
+// launches of small tiles keep more loads in flight.
+// ---------------------------------------------------------------------------
+
+// inter[t][c] = silu(W1 x) * (W3 x), 16 columns per tile: B rows 16 of W1 and
+// the same columns' 16 of W3, from w13's groups of 32 + 32 rows.
+template <typename CF>
+__global__ __launch_bounds__(CF::NW * 64) __attribute__((amdgpu_waves_per_eu(2)))
+void dense_gate_up_kernel(DenseArgs a) {
+  static_assert(CF::RN == 2, "a block of W1 and one of W3");
+  extern __shared__ float lds[];
+  const int T = a.T, H = a.H, I = a.I;
+  const int ntm = (T + CF::BM - 1) / CF::BM, ntiles = ntm * (I / 16);
+  int t = blockIdx.x;
+  if (ntiles % 8 == 0) t = (t % 8) * (ntiles / 8) + t / 8;
+  const int m0 = (t % ntm) * CF::BM, nt = t / ntm;
+  if (nt == 0) {  // the fixed routing that moe_last_routing reports
+    for (int f = threadIdx.x; f < min(CF::BM, T - m0) * kTopK; f += CF::NW * 64) {
+      const int k = f % kTopK;
+      a.s.idx[(size_t)m0 * kTopK + f] = k < kDenseChunks ? k : -1;
+      a.s.wts[(size_t)m0 * kTopK + f] = k < kDenseChunks ? 1.0f : 0.0f;
+    }
+    if (m0 == 0 && threadIdx.x < kExperts)
+      a.s.ctrl->counts[threadIdx.x] = (int)threadIdx.x < kDenseChunks ? T : 0;
+  }
+  const float *b0 = a.w13 + ((size_t)(nt / 2) * 64 + (nt % 2) * 16) * H;
+  skinny_tile<CF>(
+      lds, a.x, T, m0, H / 32, 48u * H * 4u, [&](int r) { return (r < 16 ? r : r + 16) * H; },
+      [&](int p, int &k0) {
+        k0 = p * 32;
+        return b0;
+      });
+  for (int f = threadIdx.x; f < CF::BM * 4; f += CF::NW * 64) {
+    const int row = f / 4, c4 = (f % 4) * 4;
+    if (m0 + row >= T) break;  // later rows too
+    const f32x4 w1 = skinny_sum<CF>(lds, row, c4), w3 = skinny_sum<CF>(lds, row, 16 + c4);
+    f32x4 v;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = silu(w1[j]) * w3[j];
+    st4(a.s.inter + (size_t)(m0 + row) * I + nt * 16 + c4, v);
+  }
+}
+
+// y = inter . W2^T (+ residual); w2 [chunks][H][Ic], column k of a row in chunk
+// k / Ic.
+template <typename CF>
+__global__ __launch_bounds__(CF::NW * 64) __attribute__((amdgpu_waves_per_eu(2)))
+void dense_down_kernel(DenseArgs a) {
+  extern __shared__ float lds[];
+  const int T = a.T, H = a.H, I = a.I, Ic = I / kDenseChunks;
+  const int ntm = (T + CF::BM - 1) / CF::BM, ntiles = ntm * (H / CF::BN);
+  int t = blockIdx.x;
+  if (ntiles % 8 == 0) t = (t % 8) * (ntiles / 8) + t / 8;
+  const int m0 = (t % ntm) * CF::BM, n0 = (t / ntm) * CF::BN;
+  const int ppc = Ic / 32;  // pieces per chunk
+  skinny_tile<CF>(
+      lds, a.s.inter, T, m0, I / 32, (uint32_t)CF::BN * Ic * 4u, [&](int r) { return r * Ic; },
+      [&](int p, int &k0) {
+        const int c = p / ppc;
+        k0 = (p - c * ppc) * 32;
+        return a.w2 + ((size_t)c * H + n0) * Ic;
+      });
+  for (int f = threadIdx.x; f < CF::BM * CF::RN * 4; f += CF::NW * 64) {
+    const int row = f / (CF::RN * 4), c4 = (f % (CF::RN * 4)) * 4;
+    if (m0 + row >= T) break;  // later rows too
+    f32x4 v = skinny_sum<CF>(lds, row, c4);
+    const size_t o = (size_t)(m0 + row) * H + n0 + c4;
+    if (a.residual) v = ld4(a.residual + o) + v;
+    st4(a.y + o, v);
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Weight packing (once per set_weights)
 // ---------------------------------------------------------------------------
 
@@ -3250,6 +3326,44 @@ hipError_t launch_router(const RouterArgs &a, bool from_logits, hipStream_t st) 
       hipLaunchKernelGGL((router_kernel<false, kLargeRT, 1, kLargeKC>), dim3(nb), dim3(kThreads),
                          0, st, a);
   }
+  return hipGetLastError();
+}
+
+template <typename CF>
+static void launch_gate_up(const DenseArgs &a, hipStream_t st) {
+  const int tiles = (a.T + CF::BM - 1) / CF::BM * (a.I / 16);
+  hipLaunchKernelGGL(dense_gate_up_kernel<CF>, dim3(tiles), dim3(CF::NW * 64), CF::LDS_BYTES, st, a);
+}
+
+template <typename CF>
+static void launch_down(const DenseArgs &a, hipStream_t st) {
+  const int tiles = (a.T + CF::BM - 1) / CF::BM * (a.H / CF::BN);
+  hipLaunchKernelGGL(dense_down_kernel<CF>, dim3(tiles), dim3(CF::NW * 64), CF::LDS_BYTES, st, a);
+}
+
+bool dense_skinny_supported(int H, int I) {
+  return H % 32 == 0 && I % (32 * kDenseChunks) == 0;
+}
+
+hipError_t launch_dense_skinny(const DenseArgs &a, hipStream_t st) {
+  // Sums in chains of at most 256 products, as in the streaming kernel.
+  // Token rows per tile: one block, two, or the three that 33-48 tokens fill
+  // (gate/up at 37 tokens 16 / 32 / 48 rows 42 / 44 / 38 us, at 32 tokens 35 /
+  // 31 / 38, at 154 tokens 102 / 93 / 108); the down rows' K is long, so
+  // smaller tiles balance better (one or two column blocks: 25 / 26 us at 37
+  // tokens, 47 / 41 at 128).
+  if (a.T <= 16)
+    launch_gate_up<SkinnyTile<1, 2, 4, 4, 2>>(a, st);
+  else if (a.T > 32 && a.T <= 48)
+    launch_gate_up<SkinnyTile<3, 2, 4, 3, 2>>(a, st);
+  else
+    launch_gate_up<SkinnyTile<2, 2, 4, 4, 2>>(a, st);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  if (a.T <= 64)
+    launch_down<SkinnyTile<1, 1, 8, 4, 4>>(a, st);
+  else
+    launch_down<SkinnyTile<1, 2, 8, 4, 4>>(a, st);
   return hipGetLastError();
 }
 

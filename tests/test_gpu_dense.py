@@ -69,6 +69,45 @@ def test_dense_residual_in_place(mlp, dense_weights, oracle_mod):
     np.testing.assert_allclose(dr.download(), ref, rtol=RTOL, atol=ATOL)
 
 
+# Edges of the K-split tiles that serve up to 192 tokens: 16-, 32- and 48-row
+# gate/up tiles, one and two column blocks in the down tiles.
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [2, 15, 16, 17, 33, 37, 47, 49, 65, 97, 191])
+def test_dense_few_tokens_edges(T, mlp, dense_weights, oracle_mod):
+    from final_amd import _native, hip
+    from final_amd import workloads as W
+    say(f"[dense edges] T={T}")
+    x, r = W.gen_x(T, seed=T), W.gen_x(T, seed=T + 1)
+    dx, dr, dy = (hip.DeviceArray.from_numpy(a) for a in (x, r, np.zeros_like(x)))
+    mlp.forward_gpu(dx, dy, T, residual=dr)
+    hip.synchronize()
+    ref = oracle_mod.dense_mlp(x, *dense_weights, residual=r)
+    np.testing.assert_allclose(dy.download(), ref, rtol=RTOL, atol=ATOL)
+    # the fixed routing a forward reports, whichever kernels it ran
+    idx, w, counts = np.empty((T, 4), np.int32), np.empty((T, 4), np.float32), np.empty(32, np.int32)
+    rc = _native.lib().moe_last_routing(mlp._ctx, idx.ctypes.data, w.ctypes.data, counts.ctypes.data,
+                                        None, T, None)
+    assert rc == 0
+    assert (idx == np.arange(4)).all() and (w == 1.0).all()
+    assert (counts[:4] == T).all() and not counts[4:].any()
+
+
+@pytest.mark.gpu
+def test_dense_nonfinite_rows(mlp, dense_weights):
+    """Infinities and NaN stay in their rows."""
+    from final_amd import hip
+    from final_amd import workloads as W
+    for T in (20, 300, 700):
+        x = W.gen_x(T, seed=5)
+        y0 = mlp.forward(x)
+        x[3, 7], x[11, 0] = np.inf, np.nan
+        y = mlp.forward(x)
+        assert not np.isfinite(y[3]).any() and np.isnan(y[11]).all()
+        keep = np.setdiff1d(np.arange(T), [3, 11])
+        # other rows of a tile may be computed by the other matrix instruction
+        np.testing.assert_allclose(y[keep], y0[keep], rtol=RTOL, atol=ATOL)
+
+
 @pytest.mark.gpu
 def test_dense_context_rejects_moe_calls(mlp):
     from final_amd import _native

@@ -157,21 +157,26 @@ __global__ __launch_bounds__(256) void embed_kernel(const int *ids, const float 
 // the reduction order is moe::norm_totals')
 // ---------------------------------------------------------------------------
 
-constexpr int kNormRows = 4;  // rows per block (their loads in flight together)
+// NR rows per block, their loads in flight together: four where they fill the
+// chip, one up to kNormSplitRows, where the time is one block's: a block of
+// four waits out four rows' reductions (9 rows 7.9 -> 3.3 us, 100 rows 8.0 ->
+// 3.4, 2048 rows 10.8 -> 6.9, 4096 rows 15.6 -> 13.4, 8192 rows 22.0 / 22.5).
+constexpr int kNormRows = 4, kNormSplitRows = 4096;
 
+template <int NR>
 __global__ __launch_bounds__(moe::kNormThreads) void rmsnorm_rows_kernel(
     const float *x, long long xs, const float *w, float *y, long long ys, int rows, int dim) {
-  __shared__ float s_grp[kNormRows * moe::kNormGroups], s_tot[kNormRows];
-  const int r0 = blockIdx.x * kNormRows;
-  const float *src[kNormRows];
-  float *dst[kNormRows];
+  __shared__ float s_grp[NR * moe::kNormGroups], s_tot[NR];
+  const int r0 = blockIdx.x * NR;
+  const float *src[NR];
+  float *dst[NR];
 #pragma unroll
-  for (int m = 0; m < kNormRows; ++m) {
+  for (int m = 0; m < NR; ++m) {
     const long long r = min(r0 + m, rows - 1);
     src[m] = x + r * xs;
     dst[m] = y + r * ys;
   }
-  moe::norm_rows<kNormRows>(src, dst, min(kNormRows, rows - r0), w, dim, s_grp, s_tot);
+  moe::norm_rows<NR>(src, dst, min(NR, rows - r0), w, dim, s_grp, s_tot);
 }
 
 // ---------------------------------------------------------------------------
@@ -180,7 +185,7 @@ __global__ __launch_bounds__(moe::kNormThreads) void rmsnorm_rows_kernel(
 
 constexpr int kHeadDim = 64;
 
-// One wave per token: its heads + kv_heads rows of 64 (q heads at columns
+// One wave per token (or part of it): its heads + kv_heads rows of 64 (q heads at columns
 // h*64, k heads at k_col + h*64), four rows per float4 load (16 lanes per
 // row, lane l holding elements 4(l%16)..4(l%16)+3), with the cos/sin row of
 // the token's position and both norm weights held in registers.  The norm is
@@ -196,8 +201,14 @@ constexpr int kHeadDim = 64;
 // contraction of each line is restated as fmaf(first product, -/+ second
 // product).
 constexpr int kRopeTokens = 4;   // tokens per block, one per wave
-constexpr int kRopeGroups = 16;  // groups of 4 rows a wave holds: heads + kv_heads <= 64
+constexpr int kRopeGroups = 16;  // groups of 4 rows of a token: heads + kv_heads <= 64
+// Up to kRopeSplitTokens a wave takes NG = 4 of a token's groups, grid.y the
+// others: the reductions of 10 groups in turn took longer than the loads (100
+// tokens 6.9 -> 3.7 us, 2048 10.5 -> 8.3, 8192 30.4 -> 26.5; 32768 115 / 131,
+// where each wave's own copy of the rotation row and weights tells).
+constexpr int kRopeSplitTokens = 8192;
 
+template <int NG>
 __global__ __launch_bounds__(256) void qk_norm_rope_kernel(float *qkv, int ld, const float *qw,
                                                            const float *kw, const float *cos_t,
                                                            const float *sin_t, int ntok, int seq,
@@ -206,7 +217,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(float *qkv, int ld, c
   const int lane = threadIdx.x & 63, r = lane >> 4, c4 = (lane & 15) * 4;
   const int t = blockIdx.x * kRopeTokens + (threadIdx.x >> 6);
   if (t >= ntok) return;  // whole waves; the kernel has no block barrier
-  const int ng = (per_tok + 3) >> 2;
+  const int g0 = blockIdx.y * NG, ng = min(((per_tok + 3) >> 2) - g0, NG);
+  if (ng <= 0) return;
   const int pos = t % seq;
   const f32x4 cs = moe::ld4(cos_t + (size_t)pos * kHeadDim + c4);
   const f32x4 sn = moe::ld4(sin_t + (size_t)pos * kHeadDim + c4);
@@ -216,19 +228,19 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(float *qkv, int ld, c
       __builtin_amdgcn_make_buffer_rsrc(row0, 0, ld * (int)sizeof(float), moe::kBufferRsrcWord3);
   // every load is unconditional (rows past per_tok read past the token's row:
   // zeros), so all of a token's loads are in flight together
-  f32x4 x[kRopeGroups];
-  uint32_t off[kRopeGroups];
+  f32x4 x[NG];
+  uint32_t off[NG];
 #pragma unroll
-  for (int j = 0; j < kRopeGroups; ++j) {
-    const int row = 4 * j + r;
+  for (int j = 0; j < NG; ++j) {
+    const int row = 4 * (g0 + j) + r;
     off[j] = row < per_tok ? (uint32_t)((row < heads ? row * kHeadDim : k_col + (row - heads) * kHeadDim) + c4) * 4u
                            : 0x7FFFFFF0u;
     x[j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, off[j], 0, 0));
   }
 #pragma unroll
-  for (int j = 0; j < kRopeGroups; ++j) {
+  for (int j = 0; j < NG; ++j) {
     if (j >= ng) continue;  // wave-uniform
-    const int row = 4 * j + r;
+    const int row = 4 * (g0 + j) + r;
     f32x4 sq;
 #pragma unroll
     for (int i = 0; i < 4; ++i) sq[i] = x[j][i] * x[j][i];
@@ -411,7 +423,7 @@ void attention_kernel(const float *qkv, int ld, float *out, int ldo, int seq, in
 // Short-conv mix
 // ---------------------------------------------------------------------------
 
-// One thread per (4 consecutive tokens, 4 channels): Bx = B * gate
+// One thread per (NT consecutive tokens, 4 channels): Bx = B * gate
 // (conv_transpose_split_kernel, layer.cu:377-378) of the window's rows, each
 // computed once, then per token the causal conv as the FMA chain of
 // causal_conv1d_kernel (layer.cu:397-403: sum from 0, taps k ascending, only
@@ -420,28 +432,32 @@ void attention_kernel(const float *qkv, int ld, float *out, int ldo, int seq, in
 // take neighbouring channels of the same tokens (coalesced rows); the window's
 // first L-1 rows are re-read by the thread of the previous tokens.
 constexpr int kConvTok = 4;   // tokens per thread
+// Up to here one: more threads, each with one window to wait for (9 tokens 4.9
+// -> 3.3 us, 154 tokens 5.2 -> 4.1; 512 tokens 5.6 / 7.1: windows read twice)
+constexpr int kConvSplitTokens = 256;
 constexpr int kConvMaxL = 4;  // taps the window holds
 
+template <int NT>
 __global__ __launch_bounds__(256) void shortconv_kernel(const float *bcg, const float *w, float *y,
                                                         long long T, int seq, int H, int L) {
 #pragma clang fp contract(off)
   const int H4 = H / 4;
-  const long long groups = (T + kConvTok - 1) / kConvTok;
+  const long long groups = (T + NT - 1) / NT;
   for (long long f = blockIdx.x * 256LL + threadIdx.x; f < groups * H4;
        f += (long long)gridDim.x * 256) {
     const long long tg = f / H4;
     const int c = (int)(f - tg * H4) * 4;
-    const long long t0 = tg * kConvTok;
+    const long long t0 = tg * NT;
     // taps of the 4 channels: w[c + j][k] = w[c*L + j*L + k], 4L floats from c*L
     float wk[4][kConvMaxL];
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int k = 0; k < kConvMaxL; ++k) wk[j][k] = k < L ? w[(c + j) * L + k] : 0.0f;
-    // Bx of tokens t0 - (L-1) .. t0 + kConvTok - 1 (zero where outside the tensor)
-    f32x4 bx[kConvTok + kConvMaxL - 1];
+    // Bx of tokens t0 - (L-1) .. t0 + NT - 1 (zero where outside the tensor)
+    f32x4 bx[NT + kConvMaxL - 1];
 #pragma unroll
-    for (int r = 0; r < kConvTok + kConvMaxL - 1; ++r) {
+    for (int r = 0; r < NT + kConvMaxL - 1; ++r) {
       const long long t = t0 - (kConvMaxL - 1) + r;
       if (t >= 0 && t < T && r >= kConvMaxL - L) {
         const float *row = bcg + t * 3 * H;
@@ -451,7 +467,7 @@ __global__ __launch_bounds__(256) void shortconv_kernel(const float *bcg, const 
       }
     }
 #pragma unroll
-    for (int u = 0; u < kConvTok; ++u) {
+    for (int u = 0; u < NT; ++u) {
       const long long t = t0 + u;
       if (t >= T) break;
       const int s = (int)(t % seq);
@@ -568,8 +584,12 @@ hipError_t launch_embed(const int *ids, const float *table, float *h, int T, int
 hipError_t launch_rmsnorm_rows(const float *x, long long x_stride, const float *w, float *y,
                                long long y_stride, int rows, int dim, hipStream_t st) {
   if (rows <= 0) return hipSuccess;
-  hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3((rows + kNormRows - 1) / kNormRows),
-                     dim3(moe::kNormThreads), 0, st, x, x_stride, w, y, y_stride, rows, dim);
+  if (rows <= kNormSplitRows)
+    hipLaunchKernelGGL(rmsnorm_rows_kernel<1>, dim3(rows), dim3(moe::kNormThreads), 0, st, x, x_stride,
+                       w, y, y_stride, rows, dim);
+  else
+    hipLaunchKernelGGL(rmsnorm_rows_kernel<kNormRows>, dim3((rows + kNormRows - 1) / kNormRows),
+                       dim3(moe::kNormThreads), 0, st, x, x_stride, w, y, y_stride, rows, dim);
   return hipGetLastError();
 }
 
@@ -579,8 +599,13 @@ hipError_t launch_qk_norm_rope(float *qkv, int ld, const float *qw, const float 
   const long long ntok = (long long)batch * seq;
   if (ntok <= 0) return hipSuccess;
   const long long grid = (ntok + kRopeTokens - 1) / kRopeTokens;
-  hipLaunchKernelGGL(qk_norm_rope_kernel, dim3((unsigned)grid), dim3(256), 0, st, qkv, ld, qw, kw,
-                     cos_t, sin_t, (int)ntok, seq, heads, heads + kv_heads, k_col);
+  const int per_tok = heads + kv_heads;
+  if (ntok <= kRopeSplitTokens)
+    hipLaunchKernelGGL(qk_norm_rope_kernel<4>, dim3((unsigned)grid, (per_tok + 15) / 16), dim3(256), 0,
+                       st, qkv, ld, qw, kw, cos_t, sin_t, (int)ntok, seq, heads, per_tok, k_col);
+  else
+    hipLaunchKernelGGL(qk_norm_rope_kernel<kRopeGroups>, dim3((unsigned)grid), dim3(256), 0, st, qkv, ld,
+                       qw, kw, cos_t, sin_t, (int)ntok, seq, heads, per_tok, k_col);
   return hipGetLastError();
 }
 
@@ -600,10 +625,14 @@ hipError_t launch_shortconv(const float *bcg, const float *w, float *y, int batc
   const long long T = (long long)batch * seq;
   if (T <= 0) return hipSuccess;
   if (H % 4 != 0 || L <= 0 || L > kConvMaxL) return hipErrorInvalidValue;
-  const long long n = (T + kConvTok - 1) / kConvTok * (H / 4);
+  const bool split = T <= kConvSplitTokens;
+  const long long n = (split ? T : (T + kConvTok - 1) / kConvTok) * (H / 4);
   const long long grid = std::min<long long>((n + 255) / 256, 65536);
-  hipLaunchKernelGGL(shortconv_kernel, dim3((unsigned)grid), dim3(256), 0, st, bcg, w, y, T, seq,
-                     H, L);
+  if (split)
+    hipLaunchKernelGGL(shortconv_kernel<1>, dim3((unsigned)grid), dim3(256), 0, st, bcg, w, y, T, seq, H, L);
+  else
+    hipLaunchKernelGGL(shortconv_kernel<kConvTok>, dim3((unsigned)grid), dim3(256), 0, st, bcg, w, y, T,
+                       seq, H, L);
   return hipGetLastError();
 }
 

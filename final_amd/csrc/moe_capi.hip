@@ -755,11 +755,12 @@ int moe_dense_forward(moe_ctx *ctx, const float *x, float *y, const float *resid
     ctx->routed_T = 0;
     return MOE_OK;
   }
-  if (!x || !aligned16(x)) return MOE_ERR_INVALID_ARG;
+  if (!experts_args_ok(x, y, residual)) return MOE_ERR_INVALID_ARG;
   DeviceGuard g(ctx->device);
   if (!g.ok) return MOE_ERR_HIP;
-  if (ctx_plan(ctx, num_tokens) == 0 && dense_skinny_supported(ctx->d.hidden, ctx->dense_inter) &&
-      experts_args_ok(x, y, residual)) {
+  // the streaming plan's sizes: no task queue, K-split tiles instead (the
+  // shapes it is compiled for suit them)
+  if (ctx_plan(ctx, num_tokens) == 0) {
     // the chunks' inter rows [4T][I / 4] hold the [T][I] of this path
     DenseArgs da{};
     da.x = x;
@@ -787,7 +788,7 @@ int moe_dense_forward(moe_ctx *ctx, const float *x, float *y, const float *resid
   a.H = ctx->d.hidden;
   a.inter = ctx->d.inter;
   a.tile_rows = ctx_plan(ctx, num_tokens);
-  a.bn = a.tile_rows == 0 ? stream_rows_dense(num_tokens) : expert_bn(a.tile_rows, num_tokens);
+  a.bn = expert_bn(a.tile_rows, num_tokens);
   a.tail_units = tail_units(ctx, a.tile_rows, a.bn, num_tokens);
   a.max_units = ctx->max_units;
   if (launch_router_dense(a, static_cast<hipStream_t>(stream)) != hipSuccess) return MOE_ERR_HIP;

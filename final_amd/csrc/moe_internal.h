@@ -218,7 +218,6 @@ struct DenseArgs {
   int T, H, I;
 };
 hipError_t launch_dense_skinny(const DenseArgs &a, hipStream_t st);
-bool dense_skinny_supported(int H, int I);
 // Whether the weight-streaming kernel is compiled for (H, I).
 bool stream_supported(int H, int I);
 // Largest batch the streaming plan handles (its slot -> token map is in LDS).
@@ -234,8 +233,5 @@ bool router_can_defer(int T, int tile_rows, int bn);
 // Whether a forward under an MFMA plan may route from score bounds (the
 // context's Scratch must also hold bounds and smap, and T * kExperts slots).
 bool router_can_bound(int T, int tile_rows, int H);
-// Weight rows per streaming task for the dense FFN, whose chunks all hold T
-// tokens: 32-row tasks with 4 token passes above 32 tokens.
-int stream_rows_dense(int T);
 
 }  // namespace moe

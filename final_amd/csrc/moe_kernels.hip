@@ -82,11 +82,13 @@ __device__ __forceinline__ float ref_sigmoid(float x) {
 
 // Four rows per block (their loads in flight together): out = rmsnorm(h)
 // (large batches; small ones normalise inside router_decode_kernel).
-constexpr int kNormRowsPerBlock = 4;
+// One row per block up to kNormSplitRows (the decoder's norm has the same rule
+// and the figures).
+constexpr int kNormRowsPerBlock = 4, kNormSplitRows = 4096;
 
+template <int NR>
 __global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(const float *h, const float *w,
                                                                float *out, int T, int H) {
-  constexpr int NR = kNormRowsPerBlock;
   __shared__ float s_grp[NR * kNormGroups], s_tot[NR];
   const int r0 = blockIdx.x * NR;
   const float *src[NR];
@@ -1156,15 +1158,7 @@ __global__ __launch_bounds__(kThreads) void router_dense_kernel(RouterArgs a) {
   __shared__ int s_flag;
   const int tid = threadIdx.x;
   const int T = a.T, t0 = blockIdx.x * RT;
-  // blocks past the token blocks only prepare the expert kernel's rows
   const int nb = (T + RT - 1) / RT;
-  if ((int)gridDim.x > nb) {
-    if ((int)blockIdx.x >= nb)
-      fill_unwritten(a, blockIdx.x - nb, gridDim.x - nb, tid, kThreads);
-  } else {
-    fill_unwritten(a, blockIdx.x, gridDim.x, tid, kThreads);
-  }
-  if ((int)blockIdx.x >= nb) return;
   const int nt = min(RT, T - t0);
   for (int f = tid; f < nt * kTopK; f += kThreads) {
     const size_t g = (size_t)t0 * kTopK + f;
@@ -3271,10 +3265,8 @@ bool router_fuses_norm(int T) { return T <= kSplitRouterTokens; }
 
 hipError_t launch_router_dense(const RouterArgs &a, hipStream_t st) {
   if (a.T <= 64) {
-    // the weight-streaming plan adds blocks that prepare its rows
     const int nb = (a.T + kSmallRT - 1) / kSmallRT;
-    const int grid = a.tile_rows == 0 ? nb * (1 + kDecES) : nb;
-    hipLaunchKernelGGL(router_dense_kernel<kSmallRT>, dim3(grid), dim3(kThreads), 0, st, a);
+    hipLaunchKernelGGL(router_dense_kernel<kSmallRT>, dim3(nb), dim3(kThreads), 0, st, a);
   } else {
     const int nb = (a.T + kLargeRT - 1) / kLargeRT;
     hipLaunchKernelGGL(router_dense_kernel<kLargeRT>, dim3(nb), dim3(kThreads), 0, st, a);
@@ -3284,8 +3276,12 @@ hipError_t launch_router_dense(const RouterArgs &a, hipStream_t st) {
 
 hipError_t launch_rmsnorm(const float *h, const float *w, float *out, int T, int H, hipStream_t st) {
   if (T <= 0) return hipSuccess;
-  hipLaunchKernelGGL(rmsnorm_kernel, dim3((T + kNormRowsPerBlock - 1) / kNormRowsPerBlock),
-                     dim3(kNormThreads), 0, st, h, w, out, T, H);
+  if (T <= kNormSplitRows)
+    hipLaunchKernelGGL(rmsnorm_kernel<1>, dim3(T), dim3(kNormThreads), 0, st, h, w, out, T, H);
+  else
+    hipLaunchKernelGGL(rmsnorm_kernel<kNormRowsPerBlock>,
+                       dim3((T + kNormRowsPerBlock - 1) / kNormRowsPerBlock), dim3(kNormThreads), 0, st,
+                       h, w, out, T, H);
   return hipGetLastError();
 }
 
@@ -3341,11 +3337,8 @@ static void launch_down(const DenseArgs &a, hipStream_t st) {
   hipLaunchKernelGGL(dense_down_kernel<CF>, dim3(tiles), dim3(CF::NW * 64), CF::LDS_BYTES, st, a);
 }
 
-bool dense_skinny_supported(int H, int I) {
-  return H % 32 == 0 && I % (32 * kDenseChunks) == 0;
-}
-
 hipError_t launch_dense_skinny(const DenseArgs &a, hipStream_t st) {
+  if (a.H % 32 != 0 || a.I % (32 * kDenseChunks) != 0) return hipErrorInvalidValue;
   // Sums in chains of at most 256 products, as in the streaming kernel.
   // Token rows per tile: one block, two, or the three that 33-48 tokens fill
   // (gate/up at 37 tokens 16 / 32 / 48 rows 42 / 44 / 38 us, at 32 tokens 35 /
@@ -3437,10 +3430,6 @@ hipError_t launch_experts(const ExpertArgs &a, int tile_rows, int grid,
       return hipErrorInvalidValue;
   }
   return hipGetLastError();
-}
-
-int stream_rows_dense(int T) {
-  return T > 2 * kRingTokens ? kStreamRows * kRingDenseGroups : expert_bn(0, T);
 }
 
 bool router_can_bound(int T, int tile_rows, int H) {

@@ -626,6 +626,7 @@ int moe_experts(moe_ctx *ctx, const float *x, float *y, const float *residual,
   const int plan = ctx->routed_plan;
   a.bounds = ctx->routed_bounds ? 1 : 0;
   a.tail_units = ctx->routed_tail;
+  a.split = !ctx->routed_bounds && expert_split(plan, num_tokens, ctx->dense);
   const int pi = plan_index(plan);
   if (pi < 0) return MOE_ERR_INVALID_ARG;
   // the routing (and, for the streaming plan, the rows the router prepared)
@@ -695,6 +696,7 @@ int moe_forward_noalloc(moe_ctx *ctx, const float *x, float *y, const float *res
   ea.w = ra.w;
   ea.s = s;
   ea.T = T;
+  ea.split = expert_split(ra.tile_rows, T, false);
   ea.H = ctx->d.hidden;
   ea.I = ctx->d.inter;
   ea.wait_limit = kDefaultWaitLimit / (ctx->wait_div > 0 ? ctx->wait_div : 1);

@@ -188,7 +188,18 @@ struct ExpertArgs {
   // routing's own values, so a block reads no control field before its plan)
   int bounds;
   int tail_units;
+  int split;  // 64-row plan: split-bf16 tiles (expert_split)
 };
+
+// Whether a 64-row plan's tiles run as split-bf16 tiles: when the experts hold
+// more rows than this on average.  Below, the units are padded and the 16-row
+// fp32 layouts do less work (MoE block, whole step, fp32 / split: 128 tokens
+// 268 / 296 us, 256 306 / 328, 301 345 / 357, 350 378 / 363, 400 417 / 387, 512
+// 523 / 495).
+constexpr int kSplitMinRows = 40;
+inline bool expert_split(int tile_rows, int T, bool dense) {
+  return tile_rows == 64 && (long long)T * kTopK > kSplitMinRows * (dense ? kDenseChunks : kExperts);
+}
 
 // Launchers (moe_kernels.hip).  Return hipSuccess or the launch error.
 hipError_t launch_router(const RouterArgs &a, bool from_logits, hipStream_t st);

@@ -1622,16 +1622,13 @@ __device__ __forceinline__ int first_round_left(Ctrl *c, int f) {
   return -1;
 }
 
-// The 64-row plan's full-width tiles run as split-bf16 tiles (split_tile.h)
-// when its active experts hold more rows than this on average: below, the
-// units are padded and the 16-row fp32 layouts do less work (MoE block, whole
-// step, fp32 / split: 128 tokens 268 / 296 us, 256 306 / 328, 301 345 / 357,
-// 350 378 / 363, 400 417 / 387, 512 523 / 495).
-constexpr int kSplitMinRows = 40;
+// SPLIT (64-row plan): full-width tiles run as split-bf16 tiles
+// (split_tile.h), a kernel of its own, so that small batches keep the fp32
+// tiles' registers and LDS; ExpertArgs::split says when.
 using SplitUnit = SplitTile<64, 128, 2>;
 // 128-row plan: split-bf16 tiles only, three blocks per CU (three waves per
 // SIMD in 168 registers: 4096 tokens 2139 -> 1954 us, 16384 7808 -> 7122).
-template <int BM>
+template <int BM, bool SPLIT = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(BM == 128 ? 3 : 2)))
 void expert_mfma_kernel(ExpertArgs a) {
   using TL = Tile<BM>;
@@ -1640,7 +1637,7 @@ void expert_mfma_kernel(ExpertArgs a) {
   __shared__ int s_unit_off[kExperts + 1];
   __shared__ int s_full_off[kExperts + 1];  // unit order (unit_rows)
   __shared__ int s_pexp[kExperts];
-  __shared__ int s_nfull, s_lpt, s_split;
+  __shared__ int s_nfull, s_lpt;
   __shared__ int s_offsets[kExperts + 1];
   __shared__ int s_counts[kExperts];
   __shared__ int s_aoff[BM];
@@ -1648,7 +1645,7 @@ void expert_mfma_kernel(ExpertArgs a) {
   __shared__ int s_ncomb;
   // routing from score bounds (Ctrl::deferred == 3): 32- and 64-row plans
   // of up to kBoundTokens tokens, planned by every block (bounds_local_plan)
-  constexpr bool kBounds = BM <= 64;
+  constexpr bool kBounds = BM <= 64 && !SPLIT;
   struct NoPlan {};
   __shared__ typename std::conditional<kBounds, BoundPlan, NoPlan>::type s_bp;
   Ctrl *c = a.s.ctrl;
@@ -1702,9 +1699,7 @@ void expert_mfma_kernel(ExpertArgs a) {
     int nfull;
     s_full_off[tid] = lane_scan32(cnt / BM, tid, &nfull);
     const int npart = __popcll(__ballot(part > 0));
-    const int nactive = __popcll(__ballot(cnt > 0));
     if (tid == 0) {
-      s_split = !bounds && s_offsets[kExperts] > kSplitMinRows * nactive;
       s_full_off[kExperts] = nfull;
       s_nfull = nfull;
       s_lpt = 2 * nfull <= npart;
@@ -1723,7 +1718,6 @@ void expert_mfma_kernel(ExpertArgs a) {
   __syncthreads();
   const UnitOrder uo{s_unit_off, s_full_off, s_pexp, s_counts, BM <= 64 ? s_nfull : 0,
                      BM <= 64 && s_lpt != 0};
-  const bool split = BM == 64 && s_split != 0;
   // slots written by the router: gate/up tiles need not wait for the dispatch
   // tasks, which then only clear the combine counters (down tiles wait for
   // them) and write the rows of tokens without an expert
@@ -1823,9 +1817,9 @@ void expert_mfma_kernel(ExpertArgs a) {
           const float *hrow0 = a.w.w13 + ((size_t)e * 2 * I + (size_t)nt * TH::BN) * H;
           next = mfma_tile<TH, true>(lds, a.x, xbytes, s_aoff, rows, hrow0, H, inter_out, slot0,
                                      I, nt * (TH::BN / 2), next_task);
-        } else if (split) {
+        } else if constexpr (SPLIT) {
           next = split_tile<SplitUnit, true>(lds, a.x, xbytes, s_aoff, rows, brow0, H, inter_out, slot0,
-                                            I, nt * (TL::BN / 2), next_task);
+                                             I, nt * (TL::BN / 2), next_task);
         } else {
           next = mfma_tile<TL, true>(lds, a.x, xbytes, s_aoff, rows, brow0, H, inter_out, slot0,
                                      I, nt * (TL::BN / 2), next_task);
@@ -1934,7 +1928,7 @@ void expert_mfma_kernel(ExpertArgs a) {
           else
             next = split_tile<SplitTile<128, 128>, false>(lds, abase, abytes, s_aoff, rows, brow0, I, sout_out,
                                                           slot0, H, ht * TL::BN, next_task, ready);
-        } else if (split) {
+        } else if constexpr (SPLIT) {
           next = split_tile<SplitUnit, false>(lds, abase, abytes, s_aoff, rows, brow0, I, sout_out, slot0,
                                              H, ht * TL::BN, next_task, ready);
         } else {
@@ -3378,10 +3372,8 @@ bool stream_supported(int H, int I) { return stream_fn(H, I) != nullptr; }
 
 int stream_max_tokens() { return kRingMaxSlots / kTopK; }
 
-// the 64-row plan's tiles, fp32 or split
-constexpr size_t kLds64 = std::max(Tile<64>::LDS_FLOATS * sizeof(float), SplitUnit::LDS_BYTES);
-template <int BM> static void *mfma_fn() {
-  return reinterpret_cast<void *>(&expert_mfma_kernel<BM>);
+template <int BM, bool SPLIT = false> static void *mfma_fn() {
+  return reinterpret_cast<void *>(&expert_mfma_kernel<BM, SPLIT>);
 }
 
 static hipError_t ensure_lds_attr(const void *fn, size_t bytes) {
@@ -3413,7 +3405,14 @@ hipError_t launch_experts(const ExpertArgs &a, int tile_rows, int grid,
       break;
     }
     case 64: {
-      const size_t lds = kLds64;
+      if (a.split) {
+        err = ensure_lds_attr(mfma_fn<64, true>(), SplitUnit::LDS_BYTES);
+        if (err != hipSuccess) return err;
+        hipLaunchKernelGGL((expert_mfma_kernel<64, true>), dim3(grid), dim3(kThreads),
+                           SplitUnit::LDS_BYTES, st, a);
+        break;
+      }
+      const size_t lds = Tile<64>::LDS_FLOATS * sizeof(float);
       err = ensure_lds_attr(mfma_fn<64>(), lds);
       if (err != hipSuccess) return err;
       hipLaunchKernelGGL(expert_mfma_kernel<64>, dim3(grid), dim3(kThreads), lds, st, a);
@@ -3467,7 +3466,14 @@ int expert_blocks_per_cu(int tile_rows) {
       break;
     case 64:
       e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-          &n, mfma_fn<64>(), kThreads, kLds64);
+          &n, mfma_fn<64>(), kThreads, Tile<64>::LDS_FLOATS * sizeof(float));
+      if (e == hipSuccess) {
+        // the split-bf16 form shares the grid
+        int ns = 0;
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&ns, mfma_fn<64, true>(), kThreads,
+                                                         SplitUnit::LDS_BYTES);
+        n = std::min(n, ns);
+      }
       break;
     case 128:
       e = hipOccupancyMaxActiveBlocksPerMultiprocessor(

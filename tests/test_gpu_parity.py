@@ -55,6 +55,29 @@ def test_forward_matches_oracle(T, block, real_weights, oracle_mod):
     np.testing.assert_allclose(y, ref["y"], rtol=RTOL, atol=ATOL)
 
 
+# Either side of the sizes where the 64-row plan takes split-bf16 tiles (more
+# than 320 tokens) and the 128-row plan follows it (561).
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,rows", [(320, 64), (321, 64), (440, 64), (560, 64), (561, 128), (700, 128)])
+def test_split_tile_plans(T, rows, block, real_weights, oracle_mod):
+    from final_amd import workloads as W
+    say(f"[split plans] T={T}")
+    assert block.plan(T) == rows
+    x = W.gen_x(T, seed=T)
+    y = block.forward(x)
+    ref = oracle_forward(oracle_mod, real_weights, x)
+    check_routing(block.last_routing(), ref)
+    np.testing.assert_allclose(y, ref["y"], rtol=RTOL, atol=ATOL)
+    # an infinity makes its token's outputs non-finite and no other's; the
+    # units that hold it compute in fp32
+    xi = x.copy()
+    xi[T // 2, 5] = np.inf
+    yi = block.forward(xi)
+    keep = np.arange(T) != T // 2
+    assert not np.isfinite(yi[T // 2]).all()
+    np.testing.assert_allclose(yi[keep], ref["y"][keep], rtol=RTOL, atol=ATOL)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("plan", [0, 32, 64, 128])
 def test_every_kernel_plan(plan, block, real_weights, oracle_mod):

@@ -15,10 +15,11 @@ template <int BM> struct TileCfg;
 // 4 waves as WAVES_M x WAVES_N; a wave owns WM 32-row blocks x WN 32-column
 // blocks.  B rows come in groups of 64 (gate/up phase: 32 rows of W1, then
 // the same 32 columns' rows of W3), and the epilogue pairs them through LDS.
+// (128: the shape of the 128-row plan's tiles, which split_tile.h computes)
 template <> struct TileCfg<128> {
   static constexpr int WAVES_M = 2, WM = 2, WAVES_N = 2, WN = 2, BK = 32, NS = 2;
 };
-// 64x128 tiles (49-831 tokens): 64x256 tiles left 1.4 tiles per block at
+// 64x128 tiles: 64x256 tiles left 1.4 tiles per block at
 // T=256 (637 us per step, 527 with 64x128); 64x64 tiles balance the blocks
 // better but lose more per tile (537 us at T=256, 1208 vs 1115 at T=1024)
 template <> struct TileCfg<64> {
@@ -162,37 +163,28 @@ struct SlabReady {
 //   kWide: the config's WAVES_M x WAVES_N grid of 32x32 blocks.
 //   kFull: kWide for a tile whose rows are all valid, with no row checks in
 //     its inner loop (straight-line MFMA code).
-//   kNarrow (64-row tiles whose valid rows fit the first 32-row block, and
-//     128-row tiles with 81-96 valid rows): instead of the waves of the
-//     empty row blocks idling on their SIMDs, each of the 4 waves takes one
-//     32-column block and every row block that holds rows (a 128-row tile
-//     with 3 of its 4 row blocks then costs 3/4 of a full one).
+//   kNarrow (64-row tiles whose valid rows fit the first 32-row block):
+//     instead of the waves of the empty row block idling on their SIMDs, each
+//     of the 4 waves takes one 32-column block.
 //   kSkinny1 / kSkinny2 / kSkinny3 (64-row tiles with 1-16, 17-32 or 33-48
 //     valid rows, which 32-row blocks pad to twice or 4/3 the rows):
 //     v_mfma_f32_16x16x4_f32 over 1, 2 or 3 16-row blocks, each wave taking
 //     a quarter of the columns as 16-column blocks (the 2-block form serves
 //     the half-width tiles, which the narrow layout cannot split in four).
-//     kSkinny5 / kSkinny7: the same over 5 or 7 16-row blocks, for 128-row
-//     tiles with 65-80 or 97-112 valid rows (5/8 and 7/8 of a full tile's
-//     MFMAs, where 32-row blocks take 3/4 and all of it).
 // Same tile, LDS layout and products in every layout.
-enum TileLayout {
-  kWide = 0, kNarrow = 1, kSkinny1 = 2, kSkinny3 = 3, kFull = 4, kSkinny2 = 5, kSkinny5 = 6,
-  kSkinny7 = 7
-};
+enum TileLayout { kWide = 0, kNarrow = 1, kSkinny1 = 2, kSkinny3 = 3, kFull = 4, kSkinny2 = 5 };
 
-// 64x128 tiles (the 2 x 2 grid of 32x64 wave tiles) and 128x128 tiles (2 x 2
-// of 64x64): four 32-column blocks, one per wave.  (A 128-row tile with at
-// most 64 valid rows runs as a 64-row tile; its caller decides.)
+// 64x128 tiles (the 2 x 2 grid of 32x64 wave tiles): four 32-column blocks,
+// one per wave.
 template <typename TL>
 constexpr bool tile_narrowable() {
-  return TL::WAVES_M == 2 && TL::WAVES_N == 2 && TL::WN == 2 && TL::BN == 128;
+  return TL::BM == 64 && TL::WAVES_M == 2 && TL::WAVES_N == 2 && TL::WN == 2 && TL::BN == 128;
 }
-// 64- and 128-row tiles of 4 waves whose columns split into 16-column blocks
-// per wave (64x128, the half-width 64x64, 128x128): the 16-row layouts.
+// 64-row tiles of 4 waves whose columns split into 16-column blocks per wave
+// (64x128, the half-width 64x64): the 16-row layouts.
 template <typename TL>
 constexpr bool tile_skinnyable() {
-  return (TL::BM == 64 || TL::BM == 128) && TL::WAVES_M * TL::WAVES_N == 4 && TL::BN % 64 == 0;
+  return TL::BM == 64 && TL::WAVES_M * TL::WAVES_N == 4 && TL::BN % 64 == 0;
 }
 
 // The block's next task, claimed by thread 0 at the end of a tile's MFMAs:
@@ -218,8 +210,7 @@ __device__ __forceinline__ int tile_slabs(float *lds, const uint32_t (&a_src)[TL
   constexpr int WM = TL::WM, WN = TL::WN, BK = TL::BK, PITCH = TL::PITCH;
   constexpr int A_PER = TL::A_PER, B_PER = TL::B_PER;
   constexpr int ROWS_PER_PASS = kThreads / TL::KV;
-  constexpr bool SKINNY = LAYOUT == kSkinny1 || LAYOUT == kSkinny2 || LAYOUT == kSkinny3 ||
-                          LAYOUT == kSkinny5 || LAYOUT == kSkinny7;
+  constexpr bool SKINNY = LAYOUT == kSkinny1 || LAYOUT == kSkinny2 || LAYOUT == kSkinny3;
   constexpr bool NARROW = LAYOUT == kNarrow;
   static_assert(!NARROW || tile_narrowable<TL>(), "narrow layout of 64x128 tiles");
   static_assert(!SKINNY || tile_skinnyable<TL>(), "16-row layouts of 64-row tiles");
@@ -243,8 +234,7 @@ __device__ __forceinline__ int tile_slabs(float *lds, const uint32_t (&a_src)[TL
   // skinny layout: lane l supplies row l % 16 at k offset 4 * (l / 16) of each
   // 16-wide k group, as a float4 whose component q feeds the q-th MFMA (the
   // same k permutation in A and B)
-  constexpr int SRB = LAYOUT == kSkinny7 ? 7 : LAYOUT == kSkinny5 ? 5 : LAYOUT == kSkinny3 ? 3
-                      : LAYOUT == kSkinny2 ? 2 : 1;
+  constexpr int SRB = LAYOUT == kSkinny3 ? 3 : LAYOUT == kSkinny2 ? 2 : 1;
   static_assert(SRB * 16 <= BM, "16-row blocks of the tile");
   constexpr int SKC = BN / 64;  // 16-column blocks per wave
   const int l16 = lane & 15, k16 = (lane >> 4) * 4;
@@ -435,25 +425,17 @@ __device__ __forceinline__ int mfma_tile(float *lds, const float *abase, uint32_
   const uint32_t bsrc = (uint32_t)(lrow * K + lc4) * 4u;
   const int lds_st = lrow * TL::PITCH + lc4;
 
-  constexpr bool kNa = tile_narrowable<TL>(), kSk = tile_skinnyable<TL>() && BM == 64;
-  constexpr bool kSkL = tile_skinnyable<TL>() && BM == 128;
+  constexpr bool kNa = tile_narrowable<TL>(), kSk = tile_skinnyable<TL>();
   constexpr TileLayout kS1 = kSk ? kSkinny1 : kWide, kS2 = kSk ? kSkinny2 : kWide;
   constexpr TileLayout kS3 = kSk ? kSkinny3 : kWide, kNw = kNa ? kNarrow : kWide;
-  constexpr TileLayout kS5 = kSkL ? kSkinny5 : kWide, kS7 = kSkL ? kSkinny7 : kWide;
   int next;
-  if (kSkL && rows_valid > 64 && rows_valid <= 80)
-    next = tile_slabs<TL, kS5, Ready, Claim>(lds, a_src, abase_r, bsrc_r, none_r, bsrc, lds_st, lrow, K,
-                               rows_valid, head, ready);
-  else if (kSkL && rows_valid > 96 && rows_valid <= 112)
-    next = tile_slabs<TL, kS7, Ready, Claim>(lds, a_src, abase_r, bsrc_r, none_r, bsrc, lds_st, lrow, K,
-                               rows_valid, head, ready);
-  else if (kSk && rows_valid <= 16)
+  if (kSk && rows_valid <= 16)
     next = tile_slabs<TL, kS1, Ready, Claim>(lds, a_src, abase_r, bsrc_r, none_r, bsrc, lds_st, lrow, K,
                                rows_valid, head, ready);
   else if (kSk && rows_valid > 32 && rows_valid <= 48)
     next = tile_slabs<TL, kS3, Ready, Claim>(lds, a_src, abase_r, bsrc_r, none_r, bsrc, lds_st, lrow, K,
                                rows_valid, head, ready);
-  else if (kNa && (BM == 64 ? rows_valid <= 32 : rows_valid > 80 && rows_valid <= 96))
+  else if (kNa && rows_valid <= 32)
     next = tile_slabs<TL, kNw, Ready, Claim>(lds, a_src, abase_r, bsrc_r, none_r, bsrc, lds_st, lrow, K,
                                rows_valid, head, ready);
   else if (kSk && rows_valid <= 32)

@@ -15,7 +15,9 @@
 // Values the split cannot carry (infinities, NaN, magnitudes above the largest
 // bf16, which round to infinity) leave a NaN or an infinity in every output
 // they reach, as does an fp32 overflow: a wave that finds one in its outputs
-// computes them again with the fp32 instruction.
+// computes its block again with the fp32 instruction and takes those outputs
+// from there.  The others keep theirs, so that no row's bits depend on what
+// other rows of its tile hold.
 #pragma once
 
 #include "gpu_common.h"
@@ -103,7 +105,12 @@ __device__ __forceinline__ int split_tile(float *lds, const float *abase, uint32
                                           Ready ready = Ready{}) {
   constexpr int AM = TL::AM, BM = TL::BM, PA = TL::A_PASSES, PASSES = TL::PASSES;
   uint16_t *planes = reinterpret_cast<uint16_t *>(lds);
-  const int tid = threadIdx.x, lane = tid & 63;
+  // through asm, so that the compiler cannot compute a tile's offsets outside
+  // the caller's task loop: every kind of tile's, held throughout, took the
+  // registers of the third block per CU
+  int tid = threadIdx.x;
+  asm("" : "+v"(tid));
+  const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const __amdgpu_buffer_rsrc_t ar =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(abase), 0, (int)abytes, kBufferRsrcWord3);
@@ -235,55 +242,63 @@ __device__ __forceinline__ int split_tile(float *lds, const float *abase, uint32
 
   const int next = tid == 0 ? claim_next(head) : 0;
 
-  // Results: lane l holds column l % 32 and rows 8 (r / 4) + 4 (l / 32) + r % 4
-  // of each block, so a store writes 128 contiguous bytes of two rows.
-  auto emit = [&](int i, const floatx16 &c0, const floatx16 &c1) {
+  int et = tid;  // and the epilogue's offsets not before the slab loop
+  asm("" : "+v"(et));
+  const int elr = et & 31, elh = (et >> 5) & 1;
+
+#pragma unroll
+  for (int i = 0; i < AM; ++i) {
+    int any = 0;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) any |= (int)not_finite(acc[i][0][r]) | (int)not_finite(acc[i][1][r]);
+    if (__any(any)) {
+      // fp32 MFMAs with operands straight from memory: lane l supplies row
+      // l % 32 at k offset 4 (l / 32) of each 8-wide k group
+      const int row = wm * AM * 32 + i * 32 + elr;
+      const uint32_t ao = row < rows_valid ? (uint32_t)(aoff[row] + 4 * elh) * 4u : kTileOOB;
+      const uint32_t bo = (uint32_t)((wn * 64 + elr) * K + 4 * elh) * 4u;
+      floatx16 f[2];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) f[0][r] = f[1][r] = 0.0f;
+#pragma unroll 1
+      for (int k = 0; k < K; k += 16) {
+        f32x4 av[2], bv[2][2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          av[h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ar, ao, (k + 8 * h) * 4, 0));
+#pragma unroll
+          for (int c = 0; c < 2; ++c)
+            bv[c][h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                     br, bo + (uint32_t)(c * 32 * K) * 4u, (k + 8 * h) * 4, 0));
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+              f[c] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[h][q], bv[c][h][q], f[c], 0, 0, 0);
+      }
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (not_finite(acc[i][c][r])) acc[i][c][r] = f[c][r];
+    }
+    // lane l holds column l % 32 and rows 8 (r / 4) + 4 (l / 32) + r % 4 of
+    // each block, so a store writes 128 contiguous bytes of two rows
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const int row = wm * AM * 32 + i * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
+      const int row = wm * AM * 32 + i * 32 + 8 * (r >> 2) + 4 * elh + (r & 3);
       if (row < rows_valid) {
         const size_t o = (size_t)(row0 + row) * ldo + col0;
         if (GATED) {
-          out.store1((uint32_t)((o + wn * 32 + lr) * 4), silu(c0[r]) * c1[r]);
+          out.store1((uint32_t)((o + wn * 32 + elr) * 4), silu(acc[i][0][r]) * acc[i][1][r]);
         } else {
-          out.store1((uint32_t)((o + wn * 64 + lr) * 4), c0[r]);
-          out.store1((uint32_t)((o + wn * 64 + 32 + lr) * 4), c1[r]);
+          out.store1((uint32_t)((o + wn * 64 + elr) * 4), acc[i][0][r]);
+          out.store1((uint32_t)((o + wn * 64 + 32 + elr) * 4), acc[i][1][r]);
         }
       }
-    }
-  };
-  bool bad = false;
-#pragma unroll
-  for (int i = 0; i < AM; ++i)
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) bad |= not_finite(acc[i][c][r]);
-  if (!__any(bad)) {
-#pragma unroll
-    for (int i = 0; i < AM; ++i) emit(i, acc[i][0], acc[i][1]);
-  } else {
-    // fp32 MFMAs with operands straight from memory: lane l supplies row
-    // l % 32 at k offset 4 (l / 32) of each 8-wide k group
-    const uint32_t bo = (uint32_t)((wn * 64 + lr) * K + 4 * lh) * 4u;
-    for (int i = 0; i < AM; ++i) {
-      const int row = wm * AM * 32 + i * 32 + lr;
-      const uint32_t ao = row < rows_valid ? (uint32_t)(aoff[row] + 4 * lh) * 4u : kTileOOB;
-      floatx16 c[2];
-#pragma unroll
-      for (int r = 0; r < 16; ++r) c[0][r] = c[1][r] = 0.0f;
-      for (int k = 0; k < K; k += 8) {
-        const f32x4 a = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ar, ao, k * 4, 0));
-        const f32x4 b0 = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(br, bo, k * 4, 0));
-        const f32x4 b1 = __builtin_bit_cast(
-            f32x4, __builtin_amdgcn_raw_buffer_load_b128(br, bo + (uint32_t)(32 * K) * 4u, k * 4, 0));
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          c[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q], b0[q], c[0], 0, 0, 0);
-          c[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q], b1[q], c[1], 0, 0, 0);
-        }
-      }
-      emit(i, c[0], c[1]);
     }
   }
   return next;

@@ -94,7 +94,7 @@ def test_dense_few_tokens_edges(T, mlp, dense_weights, oracle_mod):
 
 @pytest.mark.gpu
 def test_dense_nonfinite_rows(mlp, dense_weights):
-    """Infinities and NaN stay in their rows."""
+    """Infinities and NaN stay in their rows, to the last bit of the others."""
     from final_amd import hip
     from final_amd import workloads as W
     for T in (20, 300, 700):
@@ -104,8 +104,7 @@ def test_dense_nonfinite_rows(mlp, dense_weights):
         y = mlp.forward(x)
         assert not np.isfinite(y[3]).any() and np.isnan(y[11]).all()
         keep = np.setdiff1d(np.arange(T), [3, 11])
-        # other rows of a tile may be computed by the other matrix instruction
-        np.testing.assert_allclose(y[keep], y0[keep], rtol=RTOL, atol=ATOL)
+        np.testing.assert_array_equal(y[keep].view(np.uint32), y0[keep].view(np.uint32))
 
 
 @pytest.mark.gpu

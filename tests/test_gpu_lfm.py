@@ -120,6 +120,32 @@ def test_gemm_nt_values_outside_bf16(M, N):
     assert (np.abs(got[fin] - ref[fin]) <= (K + 6) * 2.0 ** -24 * mag[fin]).all()
 
 
+# Sizes that take 64- and 128-row split-bf16 tiles; 1000 and 2600 leave a partial tile.
+SPLIT_SIZES = [(1000, 6144, 96), (1000, 6144, 2048), (2600, 6144, 96), (2600, 6144, 2048)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", SPLIT_SIZES)
+def test_gemm_nt_bits_do_not_depend_on_other_rows(M, N, K):
+    """What a row or a column holds changes no bit outside it, not even in its tile."""
+    from final_amd import hip, lfm
+    say(f"[gemm rows] M={M} N={N} K={K}")
+    r = rng(M + K)
+    A = r.standard_normal((M, K), dtype=np.float32)
+    B = (0.02 * r.standard_normal((N, K), dtype=np.float32))
+    dC = hip.DeviceArray((M, N))
+    lfm.gemm_nt(dev(A), dev(B), dC, M, N, K)
+    clean = dC.download()
+    rows, cols = [3, 70, 200, M - 1], [5, N - 2]
+    A[3, 5], A[70, 40], A[200, 7], A[M - 1, 0] = np.inf, np.nan, 3.4e38, -np.inf
+    B[5, 1], B[N - 2, 9] = np.nan, 3.4e38
+    lfm.gemm_nt(dev(A), dev(B), dC, M, N, K)
+    got = dC.download()
+    assert not np.isfinite(got[[3, 70, M - 1]]).any() and np.isnan(got[:, 5]).all()
+    keep = np.setdiff1d(np.arange(M), rows), np.setdiff1d(np.arange(N), cols)
+    assert np.array_equal(bits(got[np.ix_(*keep)]), bits(clean[np.ix_(*keep)]))
+
+
 @pytest.mark.gpu
 def test_embedding_bit_exact_and_bad_ids(oracle_mod):
     from final_amd import hip, lfm

@@ -12,12 +12,13 @@
 // instruction takes K / 2: measured against 64-bit sums its error is smaller.
 // Six of them take 192 cycles per 32x32x16 block where fp32 takes 512.
 //
-// Values the split cannot carry (infinities, NaN, magnitudes above the largest
-// bf16, which round to infinity) leave a NaN or an infinity in every output
-// they reach, as does an fp32 overflow: a wave that finds one in its outputs
-// computes its block again with the fp32 instruction and takes those outputs
-// from there.  The others keep theirs, so that no row's bits depend on what
-// other rows of its tile hold.
+// Values the split cannot carry leave outputs that a wave computes again with
+// the fp32 instruction: infinities, NaN and magnitudes above the largest bf16
+// (which round to infinity) a NaN or an infinity in every output they reach, as
+// does an fp32 overflow; magnitudes below about 2^-110, whose lowest parts fall
+// under bf16's smallest subnormal, 2^-133, an output too small for its operands
+// (kSplitFloor).  The wave takes those outputs alone from its second pass, so
+// that no row's bits depend on what other rows of its tile hold.
 #pragma once
 
 #include "gpu_common.h"
@@ -57,13 +58,24 @@ __device__ __forceinline__ void split8(const f32x4 (&v)[2], bf16x8 (&out)[3]) {
   for (int q = 0; q < 3; ++q) out[q] = __builtin_bit_cast(bf16x8, p[q]);
 }
 
+// The sum of a value's parts is off by at most 2^-134 (the instruction and the
+// conversion keep subnormals), so an output by K 2^-134 (|a| + |b|), |a| and |b|
+// the largest magnitudes of its row and its column: at most 2^-25 of an output
+// of kSplitFloor K (|a| + |b|), below which it is computed again.  The maxima
+// take half an instruction per value in the staging, where the split takes 5.5.
+constexpr float kSplitFloor = 0x1p-109f;
+
 // The six products in ascending size, as (part of A, part of B).
 constexpr int kSplitProducts = 6;
 __device__ constexpr int kSplitA[kSplitProducts] = {2, 0, 1, 1, 0, 0};
 __device__ constexpr int kSplitB[kSplitProducts] = {0, 2, 1, 0, 1, 0};
 
-__device__ __forceinline__ bool not_finite(float v) {
-  return (__builtin_bit_cast(uint32_t, v) & 0x7F800000u) == 0x7F800000u;
+// max(m, |x|, |y|) and min, each one instruction; a NaN makes either a NaN.
+__device__ __forceinline__ float max_abs(float m, float x, float y) {
+  return __builtin_elementwise_maximum(__builtin_elementwise_maximum(m, fabsf(x)), fabsf(y));
+}
+__device__ __forceinline__ float min_abs(float m, float x, float y) {
+  return __builtin_elementwise_minimum(__builtin_elementwise_minimum(m, fabsf(x)), fabsf(y));
 }
 
 // Tile of BM rows x BN columns, each of the four waves AM x 2 blocks of 32x32
@@ -148,9 +160,17 @@ __device__ __forceinline__ int split_tile(float *lds, const float *abase, uint32
   };
   // (lrow + 64 i) * 32 keeps lrow's swizzle: 64 i changes neither of its bits
   uint16_t *wr = planes + lrow * TL::BK + (lq ^ split_swizzle(lrow)) * 8;
+  float mag[PASSES];  // largest magnitude this thread staged of each of its rows
+#pragma unroll
+  for (int i = 0; i < PASSES; ++i) mag[i] = 0.0f;
   auto store = [&](int set, int buf) {
 #pragma unroll
     for (int i = 0; i < PASSES; ++i) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        mag[i] = max_abs(mag[i], st[set][i][h][0], st[set][i][h][1]);
+        mag[i] = max_abs(mag[i], st[set][i][h][2], st[set][i][h][3]);
+      }
       bf16x8 p[3];
       split8(st[set][i], p);
 #pragma unroll
@@ -246,11 +266,48 @@ __device__ __forceinline__ int split_tile(float *lds, const float *abase, uint32
   asm("" : "+v"(et));
   const int elr = et & 31, elh = (et >> 5) & 1;
 
+  // The rows' magnitudes, in LDS (free after the last barrier): A rows, then
+  // B rows, from the four threads that staged each.
+#pragma unroll
+  for (int i = 0; i < PASSES; ++i) {
+    mag[i] = __builtin_elementwise_maximum(mag[i], __shfl_xor(mag[i], 1));
+    mag[i] = __builtin_elementwise_maximum(mag[i], __shfl_xor(mag[i], 2));
+    // an output of a zero row or column is zero: no limit
+    if ((et & 3) == 0)
+      lds[(et >> 2) + 64 * i] = mag[i] != 0.0f ? mag[i] * ((float)K * kSplitFloor) : -__builtin_inff();
+  }
+  __syncthreads();
+
+  // Elements the parts do not give: not finite, or below the limit of their
+  // row and column (kSplitFloor).
+  const float mb[2] = {lds[BM + wn * 64 + elr], lds[BM + wn * 64 + 32 + elr]};
+  auto lost = [&](int i, int c, int r) {
+    const float ma = lds[wm * AM * 32 + i * 32 + 8 * (r >> 2) + 4 * elh + (r & 3)];
+    const float v = fabsf(acc[i][c][r]);
+    return !(v >= ma + mb[c] && v <= __FLT_MAX__);
+  };
 #pragma unroll
   for (int i = 0; i < AM; ++i) {
-    int any = 0;
+    // a lane's smallest results against the largest limit, then each its own
+    float top = 0.0f, ma = -__builtin_inff(), low[2] = {__builtin_inff(), __builtin_inff()};
 #pragma unroll
-    for (int r = 0; r < 16; ++r) any |= (int)not_finite(acc[i][0][r]) | (int)not_finite(acc[i][1][r]);
+    for (int q = 0; q < 4; ++q) {
+      const f32x4 m = ld4(lds + wm * AM * 32 + i * 32 + 8 * q + 4 * elh);
+      ma = fmaxf(fmaxf(ma, fmaxf(m[0], m[1])), fmaxf(m[2], m[3]));
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int h = 0; h < 4; h += 2) {
+          low[c] = min_abs(low[c], acc[i][c][4 * q + h], acc[i][c][4 * q + h + 1]);
+          top = max_abs(top, acc[i][c][4 * q + h], acc[i][c][4 * q + h + 1]);
+        }
+    }
+    bool any = !(top <= __FLT_MAX__ && low[0] >= ma + mb[0] && low[1] >= ma + mb[1]);
+    if (__any(any)) {
+      any = false;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) any = any || lost(i, 0, r) || lost(i, 1, r);
+    }
     if (__any(any)) {
       // fp32 MFMAs with operands straight from memory: lane l supplies row
       // l % 32 at k offset 4 (l / 32) of each 8-wide k group
@@ -283,7 +340,7 @@ __device__ __forceinline__ int split_tile(float *lds, const float *abase, uint32
       for (int c = 0; c < 2; ++c)
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-          if (not_finite(acc[i][c][r])) acc[i][c][r] = f[c][r];
+          if (lost(i, c, r)) acc[i][c][r] = f[c][r];
     }
     // lane l holds column l % 32 and rows 8 (r / 4) + 4 (l / 32) + r % 4 of
     // each block, so a store writes 128 contiguous bytes of two rows

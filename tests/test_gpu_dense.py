@@ -108,6 +108,28 @@ def test_dense_nonfinite_rows(mlp, dense_weights):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T", [100, 300, 700])
+def test_dense_small_inputs(T):
+    """Inputs near the smallest normal value against weights that undo them: as the same block unscaled."""
+    from final_amd import DenseMLP
+    h, i = 256, 1024
+    r = np.random.default_rng(T)
+    w = [np.float32(0.05) * r.standard_normal(s, dtype=np.float32) for s in ((i, h), (i, h), (h, i))]
+    x = r.uniform(1.0, 2.0, (T, h)).astype(np.float32)
+    ys = []
+    for e in (0, 124):
+        m = DenseMLP(h, i, max_tokens=T)
+        m.set_weights(np.ldexp(w[0], e), np.ldexp(w[1], e), w[2])
+        ys.append(m.forward(np.ldexp(x, -e)))
+        m.close()
+    # every product is the same number on both sides; each side's sums take at
+    # most h and i roundings of 2^-24, those of gate and up carried through the
+    # product and the down rows: (2 h + i) 2^-24 in the norm, and far less when
+    # roundings cancel, as they do for all but a constant sign
+    assert np.linalg.norm(ys[1] - ys[0]) <= 2 * (2 * h + i) * 2.0 ** -24 / np.sqrt(h) * np.linalg.norm(ys[0])
+
+
+@pytest.mark.gpu
 def test_dense_context_rejects_moe_calls(mlp):
     from final_amd import _native
     L = _native.lib()

@@ -147,6 +147,35 @@ def test_gemm_nt_bits_do_not_depend_on_other_rows(M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", SPLIT_SIZES)
+def test_gemm_nt_small_values(M, N, K):
+    """Operands down to the smallest subnormal, against large and small ones."""
+    from final_amd import hip, lfm
+    say(f"[gemm small] M={M} N={N} K={K}")
+    r = rng(M + K + 1)
+    A = r.standard_normal((M, K), dtype=np.float32)
+    B = r.standard_normal((N, K), dtype=np.float32)
+    # powers of two on rows of A and columns of the product: exact, but for
+    # operands that become subnormal
+    ea = np.array([0, -60, -105, -112, -118, -122, -126, -135, -148])[np.arange(M) % 9]
+    eb = np.array([0, 100, 60, -112, -124, 20, -140])[np.arange(N) % 7]
+    A = np.ldexp(A, ea[:, None]).astype(np.float32)
+    B = np.ldexp(B, eb[:, None]).astype(np.float32)
+    A[4], B[8] = 0.0, 0.0
+    A[13, ::2] = 1.0  # tiny and ordinary values in one row
+    dC = hip.DeviceArray((M, N))
+    lfm.gemm_nt(dev(A), dev(B), dC, M, N, K)
+    got = dC.download()
+    cols = np.unique(np.concatenate([np.arange(16), r.integers(0, N, 200)]))
+    ref = A.astype(np.float64) @ B[cols].astype(np.float64).T
+    # as in test_gemm_nt_dispatch_edges, and K roundings to the subnormal grid
+    tol = ((K + 6) * 2.0 ** -24 * (np.abs(A).astype(np.float64) @ np.abs(B[cols]).astype(np.float64).T)
+           + K * 2.0 ** -149)
+    bad = np.abs(got[:, cols] - ref) > tol
+    assert not bad.any(), (np.unique(ea[bad.any(1)]), np.unique(eb[cols][bad.any(0)]))
+
+
+@pytest.mark.gpu
 def test_embedding_bit_exact_and_bad_ids(oracle_mod):
     from final_amd import hip, lfm
     V, H, T = 1000, 2048, 300

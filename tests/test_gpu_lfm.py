@@ -67,7 +67,9 @@ def test_gemm_nt(M, N, K, res, oracle_mod):
                                    (113, 3072, 160), (97, 6144, 64), (333, 6144, 1056),
                                    (65, 32768, 32), (64, 32768, 96), (1000, 6144, 2048),
                                    (1009, 6144, 96), (2049, 6144, 32), (2049, 6144, 96),
-                                   (2720, 6144, 1792)])
+                                   (2720, 6144, 1792), (9, 6144, 1056), (49, 2048, 96),
+                                   (33, 6144, 1056), (9, 65536, 96), (2561, 6144, 32),
+                                   (2561, 6144, 96)])
 @pytest.mark.parametrize("res", [False, True])
 def test_gemm_nt_dispatch_edges(M, N, K, res):
     from final_amd import hip, lfm
@@ -93,7 +95,7 @@ def test_gemm_nt_dispatch_edges(M, N, K, res):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N", [(40, 2048), (100, 3072), (65, 32768), (2049, 6144)])
+@pytest.mark.parametrize("M,N", [(40, 2048), (100, 3072), (65, 32768), (2049, 6144), (2561, 6144)])
 def test_gemm_nt_values_outside_bf16(M, N):
     """Infinities, NaN and finite values above the largest bf16 give what fp32 arithmetic gives."""
     from final_amd import hip, lfm

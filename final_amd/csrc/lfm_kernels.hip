@@ -537,12 +537,14 @@ template <bool RES>
 static hipError_t gemm_dispatch(const GemmArgs &g, hipStream_t st) {
   // The kernel whose tiles are expected to take the least time (us): a launch,
   // and the longest of its rounds of blocks over the CUs, of one block alone
-  // (64- and 128-row tiles; K split over waves, a round is that), and of reading
-  // B at the rate its loads reach.  Rounds grow with K from a fixed part: with
+  // (64- and 128-row tiles, with the other CUs busy too), and of reading B at
+  // the rate its loads reach.  Rounds grow with K from a fixed part: with
   // K = 2048's times at every K, 512 x 6144 x 256 took 36 us where 64-row tiles
-  // take 18.  Fitted to 700 sizes, of which it takes 1 % longer than the best of
-  // the five on average.  Some (us; tiles 16x16 / 16x32 / 32x32 with K split
-  // over waves, 64x128 / 128x128):
+  // take 18.  Fitted to 850 sizes, of which it takes 1 % longer than the best of
+  // the five on average.  Between 16x16 and 32x32 at up to 16 rows of the LM
+  // head the rates are set for 16x16, whose sums over 8 waves, not 4, are half as
+  // long (error against 64 bits 2.9e-7, 4.1e-7).  Some (us; tiles 16x16 / 16x32 /
+  // 32x32 with K split over waves, 64x128 / 128x128):
   //   M=9    N=2048  K=2048     6.7 /  9.4 /  14 /   74 /  108
   //   M=9    N=6144  K=2048    11.3 / 12.1 /  15 /   74 /  110
   //   M=9    N=6144  K=7168    39   / 35   /  43 /  256 /  369
@@ -550,6 +552,7 @@ static hipError_t gemm_dispatch(const GemmArgs &g, hipStream_t st) {
   //   M=154  N=6144  K=2048    55   / 49   /  42 /   76 /  108
   //   M=333  N=6144  K=2048   104   / 89   /  80 /   89 /  109
   //   M=333  N=6144  K=256     61   / 50   /  27 /   17 /   20
+  //   M=896  N=2048  K=2048     -   /   -  /  70 /   77 /  109
   //   M=9    N=65536 K=2048   102   / 109  /  96 /  127 /  179
   //   M=64   N=65536 K=2048   276   / 226  / 177 /  137 /  187
   //   M=2664 N=2048  K=2048   368   / 256  / 215 /  154 /  162
@@ -559,11 +562,11 @@ static hipError_t gemm_dispatch(const GemmArgs &g, hipStream_t st) {
     return (double)(((g.M + bm - 1) / bm * (g.N / bn) + kGemmCUs - 1) / kGemmCUs);
   };
   const double cost[5] = {
-      2.9 + std::max(rounds(16, 16) * (1.0 + 0.0017 * K), b_us / 5.55),
+      2.9 + std::max(rounds(16, 16) * (1.0 + 0.0017 * K), b_us / 5.7),
       2.8 + std::max(rounds(16, 32) * (1.8 + 0.0024 * K), b_us / 4.8),
       3.8 + std::max(rounds(32, 32) * (1.4 + 0.0043 * K), b_us / 5.65),
-      4.0 + std::max({rounds(64, 128) * (0.7 + 0.0245 * K), 0.0343 * K, b_us / 4.1}),
-      6.0 + std::max({rounds(128, 128) * (1.0 + 0.0435 * K), 0.0502 * K, b_us / 3.2})};
+      4.0 + std::max({rounds(64, 128) * (0.7 + 0.0245 * K), 0.0375 * K, b_us / 4.1}),
+      6.0 + std::max({rounds(128, 128) * (1.0 + 0.0425 * K), 0.0502 * K, b_us / 3.2})};
   switch (std::min_element(cost, cost + 5) - cost) {
     case 0: return gemm_skinny_launch<1, 1, 8, 4, RES>(g, st);
     case 1: return gemm_skinny_launch<1, 2, 8, 4, RES>(g, st);

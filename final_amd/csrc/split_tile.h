@@ -78,6 +78,12 @@ __device__ __forceinline__ float min_abs(float m, float x, float y) {
   return __builtin_elementwise_minimum(__builtin_elementwise_minimum(m, fabsf(x)), fabsf(y));
 }
 
+// v of another lane of the quad.
+template <int CTRL> __device__ __forceinline__ float quad_perm(float v) {
+  return __builtin_bit_cast(
+      float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+
 // Tile of BM rows x BN columns, each of the four waves AM x 2 blocks of 32x32
 // (BN = 128: 2 x 2 waves, BN = 64: 4 x 1).  Slabs of 32 k: thread t stages 8
 // floats of rows t / 4 + 64 i (two float4s, 16 k apart, so four threads read
@@ -267,11 +273,11 @@ __device__ __forceinline__ int split_tile(float *lds, const float *abase, uint32
   const int elr = et & 31, elh = (et >> 5) & 1;
 
   // The rows' magnitudes, in LDS (free after the last barrier): A rows, then
-  // B rows, from the four threads that staged each.
+  // B rows, from the four threads that staged each (lanes ^ 1, ^ 2).
 #pragma unroll
   for (int i = 0; i < PASSES; ++i) {
-    mag[i] = __builtin_elementwise_maximum(mag[i], __shfl_xor(mag[i], 1));
-    mag[i] = __builtin_elementwise_maximum(mag[i], __shfl_xor(mag[i], 2));
+    mag[i] = __builtin_elementwise_maximum(mag[i], quad_perm<0xB1>(mag[i]));
+    mag[i] = __builtin_elementwise_maximum(mag[i], quad_perm<0x4E>(mag[i]));
     // an output of a zero row or column is zero: no limit
     if ((et & 3) == 0)
       lds[(et >> 2) + 64 * i] = mag[i] != 0.0f ? mag[i] * ((float)K * kSplitFloor) : -__builtin_inff();

@@ -194,17 +194,29 @@ static int plan_index(int rows) {
 // moe_experts, which keep the full router, take the same plans (with it,
 // streaming led up to 48).
 constexpr int kStreamMaxTokens = 10;
-// The dense FFN's 4 chunk experts each hold every token: streaming up to 192
-// tokens, 64-row split-bf16 tiles up to 640 (321 vs 372 us for 128-row tiles
-// at 512), 128-row tiles above (448 vs 420 at 768).
-static int auto_plan(int T, bool stream_ok, bool dense) {
-  if (T <= (dense ? 192 : kStreamMaxTokens) && stream_ok) return 0;
-  if (T < (dense ? 641 : 561)) return 64;
-  return 128;
+// The dense FFN, whose 4 chunk experts each hold every token: plan 0 is two
+// K-split GEMMs (launch_dense_skinny, any shape moe_dense_create takes), up to
+// 192 tokens and the work of 192 tokens at 2048 x 7168, 64-row split-bf16 tiles
+// up to 640 tokens (338 vs 394 us for 128-row tiles at 512, 400 / 409 at 640),
+// 128-row tiles above (456 vs 442 at 768).  Few tokens against 64-row tiles, us
+// (2048 x 7168: 64 tokens 85 / 147, 128 132 / 160, 160 169 / 179, 176 186 / 181,
+// 192 190 / 184, 256 241 / 222; 1024 x 4096: 192 62 / 100; 512 x 2048: 192 22 /
+// 57; 4096 x 8192: 64 158 / 223, 100 255 / 237; 4096 x 16384: 33 233 / 232, 64
+// 307 / 265): by time the line lies at 165 tokens' work, 3 % below the 192 of
+// moe_plan_tile_rows' callers.
+constexpr int kDenseFewTokens = 192;
+constexpr double kDenseFewWork = 192.0 * 2048 * 7168;
+static int auto_plan(const moe_ctx *ctx, int T) {
+  if (ctx->dense) {
+    if (T <= kDenseFewTokens && (double)T * ctx->d.hidden * ctx->dense_inter <= kDenseFewWork) return 0;
+    return T < 641 ? 64 : 128;
+  }
+  if (T <= kStreamMaxTokens && ctx->stream_ok) return 0;
+  return T < 561 ? 64 : 128;
 }
 
 static int ctx_plan(const moe_ctx *ctx, int T) {
-  const int p = ctx->tile_override >= 0 ? ctx->tile_override : auto_plan(T, ctx->stream_ok, ctx->dense);
+  const int p = ctx->tile_override >= 0 ? ctx->tile_override : auto_plan(ctx, T);
   // the streaming plan keeps the batch's slot -> token map in LDS
   return p == 0 && T > stream_max_tokens() ? 64 : p;
 }
@@ -760,9 +772,7 @@ int moe_dense_forward(moe_ctx *ctx, const float *x, float *y, const float *resid
   if (!experts_args_ok(x, y, residual)) return MOE_ERR_INVALID_ARG;
   DeviceGuard g(ctx->device);
   if (!g.ok) return MOE_ERR_HIP;
-  // the streaming plan's sizes: no task queue, K-split tiles instead (the
-  // shapes it is compiled for suit them)
-  if (ctx_plan(ctx, num_tokens) == 0) {
+  if (ctx_plan(ctx, num_tokens) == 0) {  // K-split tiles, no task queue
     // the chunks' inter rows [4T][I / 4] hold the [T][I] of this path
     DenseArgs da{};
     da.x = x;

@@ -139,9 +139,8 @@ int moe_route_logits(moe_ctx *ctx, const float *logits, int num_tokens,
  * (layer.cu:1216-1228) and its missing scratch (the reference never allocates
  * temp_buf_gpu_, layer.cu:1237).  The context runs the MoE kernels with the
  * intermediate dimension cut into 4 chunks, every token sent to all four with
- * weight 1: hidden % 256 == 0 and inter % 1024 == 0 (inter / 4 == 1792 at
- * hidden 2048 gets the weight-streaming kernel for small batches).  Release
- * with moe_destroy.  moe_forward / moe_route / moe_set_weights reject a dense
+ * weight 1; few tokens (moe_plan_tile_rows 0) run as two K-split GEMMs
+ * instead.  hidden % 256 == 0 and inter % 1024 == 0.  Release with moe_destroy.  moe_forward / moe_route / moe_set_weights reject a dense
  * context and moe_dense_* reject a MoE context. */
 int moe_dense_create(int hidden, int inter, int max_tokens, moe_ctx **out);
 
@@ -220,7 +219,8 @@ int moe_device_status(moe_ctx *ctx, moe_stream_t stream);
 int moe_last_plan_counts(moe_ctx *ctx, int *counts, moe_stream_t stream);
 
 /* Which expert kernel moe_forward picks for num_tokens: 0 = weight-streaming
- * (small T), 32/64/128 = MFMA grouped GEMM with that many rows per tile. */
+ * (small T; a dense context: K-split GEMMs), 32/64/128 = MFMA grouped GEMM with
+ * that many rows per tile. */
 int moe_plan_tile_rows(const moe_ctx *ctx, int num_tokens);
 
 /* Overrides the plan (tests): rows = -1 automatic, 0 streaming, 32/64/128.

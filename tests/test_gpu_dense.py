@@ -44,8 +44,7 @@ def test_dense_matches_oracle(T, mlp, dense_weights, oracle_mod):
     from final_amd import workloads as W
     say(f"[dense] T={T} plan={mlp.plan(T)}")
     if T <= 192:
-        # weight streaming, 4 chunks of 1792; above 64 tokens in several
-        # 64-token groups per task
+        # K-split tiles on the 4 chunks of 1792
         assert mlp.plan(T) == 0
     x = W.gen_x(T, seed=31)
     y = mlp.forward(x)
@@ -105,6 +104,40 @@ def test_dense_nonfinite_rows(mlp, dense_weights):
         assert not np.isfinite(y[3]).any() and np.isnan(y[11]).all()
         keep = np.setdiff1d(np.arange(T), [3, 11])
         np.testing.assert_array_equal(y[keep].view(np.uint32), y0[keep].view(np.uint32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("h,i", [(256, 1024), (512, 3072), (1024, 1024), (2304, 6144)])
+def test_dense_other_shapes(h, i, oracle_mod):
+    """K-split tiles for few tokens whatever the shape, against the oracle and the 64-row plan."""
+    from final_amd import DenseMLP, _native
+    r = np.random.default_rng(h + i)
+    w = [np.float32(0.04) * r.standard_normal(s, dtype=np.float32) for s in ((i, h), (i, h), (h, i))]
+    m = DenseMLP(h, i, max_tokens=200)
+    try:
+        m.set_weights(*w)
+        for T in (1, 16, 17, 33, 48, 65, 192):
+            say(f"[dense shapes] {h} x {i} T={T}")
+            x = r.standard_normal((T, h), dtype=np.float32)
+            assert m.plan(T) == 0 and m.plan(193) == 64
+            y = m.forward(x)
+            assert _native.lib().moe_force_tile_rows(m._ctx, 64) == 0
+            y64 = m.forward(x)
+            assert _native.lib().moe_force_tile_rows(m._ctx, -1) == 0
+            np.testing.assert_allclose(y, oracle_mod.dense_mlp(x, *w), rtol=RTOL, atol=ATOL)
+            np.testing.assert_allclose(y, y64, rtol=RTOL, atol=ATOL)
+        # compiled for no such shape: the forced streaming plan stays refused
+        assert _native.lib().moe_force_tile_rows(m._ctx, 0) != 0
+    finally:
+        m.close()
+
+
+@pytest.mark.gpu
+def test_dense_plan_by_work():
+    from final_amd import DenseMLP
+    m = DenseMLP(4096, 16384, max_tokens=64)
+    assert [m.plan(T) for T in (1, 42, 43, 64)] == [0, 0, 64, 64]
+    m.close()
 
 
 @pytest.mark.gpu

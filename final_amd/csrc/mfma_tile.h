@@ -15,10 +15,6 @@ template <int BM> struct TileCfg;
 // 4 waves as WAVES_M x WAVES_N; a wave owns WM 32-row blocks x WN 32-column
 // blocks.  B rows come in groups of 64 (gate/up phase: 32 rows of W1, then
 // the same 32 columns' rows of W3), and the epilogue pairs them through LDS.
-// (128: the shape of the 128-row plan's tiles, which split_tile.h computes)
-template <> struct TileCfg<128> {
-  static constexpr int WAVES_M = 2, WM = 2, WAVES_N = 2, WN = 2, BK = 32, NS = 2;
-};
 // 64x128 tiles: 64x256 tiles left 1.4 tiles per block at
 // T=256 (637 us per step, 527 with 64x128); 64x64 tiles balance the blocks
 // better but lose more per tile (537 us at T=256, 1208 vs 1115 at T=1024)
@@ -32,9 +28,6 @@ template <> struct TileCfg<32> {
 // Half-width down tiles for the last units of a launch (same rows, half the
 // columns), so the last round of tiles is half as long.
 template <int BM> struct TileHalfCfg;
-template <> struct TileHalfCfg<128> {
-  static constexpr int WAVES_M = 4, WM = 1, WAVES_N = 1, WN = 2, BK = 32, NS = 3;
-};
 template <> struct TileHalfCfg<64> {
   static constexpr int WAVES_M = 2, WM = 1, WAVES_N = 2, WN = 1, BK = 32, NS = 3;
 };

@@ -35,7 +35,7 @@ constexpr int kStreamWideTokens = 32;  // batches from this size use 64-row task
 constexpr int kRingTokens = 16;
 constexpr int kRingMaxPasses = 2;
 constexpr int kRingWideGroups = 4;
-constexpr int kRingDenseGroups = 2, kRingDensePasses = 4;
+constexpr int kRingTallGroups = 2, kRingTallPasses = 4;
 // Units (experts) whose down rows the streaming plan splits into 16-row tasks
 // at the end of the queue when its 64-row tasks are streamed in sub-groups
 // (T=64: 277 us with none, 275.7 with 2, 274.4 with 6, 277.4 with 12).

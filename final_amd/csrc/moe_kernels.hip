@@ -11,11 +11,12 @@
 //   2. expert kernel -- persistent, gate/up projection with the SwiGLU
 //      epilogue (layer.cu:773-972), down projection (layer.cu:974-1126) and
 //      the weighted top-4 combine with the residual add (layer.cu:695-721,
-//      1860-1880).  T > 48: expert_mfma_kernel, MFMA 32x32x2 f32 tiles with
-//      slots assigned by the router up to 1024 tokens, by a dispatch phase
-//      above (both replace moe_scatter_kernel, layer.cu:501-542, without
-//      copying x), one dynamic task queue, the combine inside the down
-//      tiles; 64-row tiles up to 831 tokens, 128-row tiles above.  T <= 48:
+//      1860-1880).  T > 10: expert_mfma_kernel, MFMA tiles with slots
+//      assigned by the router up to 1024 tokens, by a dispatch phase above
+//      (both replace moe_scatter_kernel, layer.cu:501-542, without copying
+//      x), one dynamic task queue, the combine inside the down tiles; 64-row
+//      fp32 tiles (mfma_tile.h) up to 320 tokens, 64-row split-bf16 tiles
+//      (split_tile.h) up to 560, 128-row split-bf16 tiles above.  T <= 10:
 //      expert_ring_kernel, weight streaming through MFMA 16x16x4 f32 with
 //      round-robin tasks and slots assigned by the router -- or, for a fused
 //      forward of at most 8 tokens, planned by each of its own blocks from
@@ -288,7 +289,7 @@ __device__ void router_plan(const RouterArgs &a, int nb, int T, PlanShared &ps,
       // experts of up to 64 tokens read each weight row once.
       int rows = a.bn;
       if (tr == 0 && rows == kStreamRows * kRingWideGroups && maxcnt > kRingMaxPasses * kRingTokens)
-        rows = kStreamRows * kRingDenseGroups;
+        rows = kStreamRows * kRingTallGroups;
       const int p1u = a.inter / (rows / 2);
       const int p2u = a.H / rows;
       ctrl->stream_rows = tr > 0 ? 0 : rows;
@@ -1624,14 +1625,17 @@ __device__ __forceinline__ int first_round_left(Ctrl *c, int f) {
 
 // SPLIT (64-row plan): full-width tiles run as split-bf16 tiles
 // (split_tile.h), a kernel of its own, so that small batches keep the fp32
-// tiles' registers and LDS; ExpertArgs::split says when.
+// tiles' registers and LDS; expert_split (moe_internal.h) says when.
 using SplitUnit = SplitTile<64, 128, 2>;
+// A plan's tiles of a unit's full and half column width.
+template <int BM> using UnitTile = std::conditional_t<BM == 128, SplitTile<128, 128>, Tile<BM>>;
+template <int BM> using UnitHalf = std::conditional_t<BM == 128, SplitTile<128, 64>, TileHalf<BM>>;
 // 128-row plan: split-bf16 tiles only, three blocks per CU (three waves per
 // SIMD in 168 registers: 4096 tokens 2139 -> 1954 us, 16384 7808 -> 7122).
 template <int BM, bool SPLIT = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(BM == 128 ? 3 : 2)))
 void expert_mfma_kernel(ExpertArgs a) {
-  using TL = Tile<BM>;
+  using TL = UnitTile<BM>;
   extern __shared__ float lds[];
   __shared__ int s_task;
   __shared__ int s_unit_off[kExperts + 1];
@@ -1641,7 +1645,7 @@ void expert_mfma_kernel(ExpertArgs a) {
   __shared__ int s_offsets[kExperts + 1];
   __shared__ int s_counts[kExperts];
   __shared__ int s_aoff[BM];
-  __shared__ int s_comb[BM * (Tile<BM>::BN / kCombineCols)];
+  __shared__ int s_comb[BM * (UnitTile<BM>::BN / kCombineCols)];
   __shared__ int s_ncomb;
   // routing from score bounds (Ctrl::deferred == 3): 32- and 64-row plans
   // of up to kBoundTokens tokens, planned by every block (bounds_local_plan)
@@ -1810,7 +1814,7 @@ void expert_mfma_kernel(ExpertArgs a) {
       const uint32_t xbytes = (uint32_t)((size_t)a.T * H * sizeof(float));
       // a 128-row unit holding at most 64 rows runs as a 64x128 tile (same
       // columns and outputs, half the padding MFMAs)
-      static_assert(Tile<64>::BN == Tile<128>::BN, "a 64-row tile covers a 128-row unit's columns");
+      static_assert(SplitTile<64, 128>::BN == UnitTile<128>::BN, "a 64-row tile covers a 128-row unit's columns");
       if constexpr (BM == 64) {
         if (ghalf) {  // one W1/W3 row group: 32 intermediate columns
           using TH = TileHalf<64>;
@@ -1824,14 +1828,13 @@ void expert_mfma_kernel(ExpertArgs a) {
           next = mfma_tile<TL, true>(lds, a.x, xbytes, s_aoff, rows, brow0, H, inter_out, slot0,
                                      I, nt * (TL::BN / 2), next_task);
         }
-      } else if (BM == 128 && ghalf) {  // one W1/W3 row group: 32 intermediate columns
-        static_assert(TileHalf<64>::BN == TileHalf<128>::BN, "a half tile's columns");
-        using TH = SplitTile<128, 64>;
-        const float *hrow0 = a.w.w13 + ((size_t)e * 2 * I + (size_t)nt * TH::BN) * H;
-        next = split_tile<TH, true>(lds, a.x, xbytes, s_aoff, rows, hrow0, H, inter_out, slot0, I,
-                                    nt * (TH::BN / 2), next_task);
-      } else if (BM == 128) {
-        if (rows <= 64)
+      } else if constexpr (BM == 128) {
+        if (ghalf) {  // one W1/W3 row group: 32 intermediate columns
+          using TH = UnitHalf<128>;
+          const float *hrow0 = a.w.w13 + ((size_t)e * 2 * I + (size_t)nt * TH::BN) * H;
+          next = split_tile<TH, true>(lds, a.x, xbytes, s_aoff, rows, hrow0, H, inter_out, slot0, I,
+                                      nt * (TH::BN / 2), next_task);
+        } else if (rows <= 64)
           next = split_tile<SplitTile<64, 128>, true>(lds, a.x, xbytes, s_aoff, rows, brow0, H, inter_out,
                                                       slot0, I, nt * (TL::BN / 2), next_task);
         else
@@ -1872,8 +1875,7 @@ void expert_mfma_kernel(ExpertArgs a) {
       // per-slab form was 0.5 % slower there), and in the 128-row plan, whose
       // slab loop has no registers to spare, the tile waits for all of them
       // first.
-      static_assert(TL::BK == TileHalf<BM>::BK && (BM != 128 || Tile<64>::BK == TL::BK),
-                    "one slab width");
+      static_assert(TL::BK == UnitHalf<BM>::BK, "one slab width");
       using Ready = typename std::conditional<BM == 128, NoWait, SlabReady>::type;
       Ready ready{};
       const bool whole = BM == 128 || a.T <= kSlabWaitMinTokens;
@@ -1899,10 +1901,10 @@ void expert_mfma_kernel(ExpertArgs a) {
         // a gate/up tile writes BN / 2 intermediate columns (a power of two,
         // at least a slab's BK): slab s needs tile s >> shift
         constexpr int kFullShift = __builtin_ctz(TL::BN / 2 / TL::BK);
-        constexpr int kHalfShift = __builtin_ctz(TileHalf<BM>::BN / 2 / TL::BK);
-        static_assert((TL::BN / 2) % TL::BK == 0 && (TileHalf<BM>::BN / 2) % TL::BK == 0 &&
+        constexpr int kHalfShift = __builtin_ctz(UnitHalf<BM>::BN / 2 / TL::BK);
+        static_assert((TL::BN / 2) % TL::BK == 0 && (UnitHalf<BM>::BN / 2) % TL::BK == 0 &&
                           (1 << kFullShift) * TL::BK == TL::BN / 2 &&
-                          (1 << kHalfShift) * TL::BK == TileHalf<BM>::BN / 2,
+                          (1 << kHalfShift) * TL::BK == UnitHalf<BM>::BN / 2,
                       "gate/up tiles cover whole slabs");
         ready = Ready{a.s.dep + (size_t)dep_words(I) * u, u >= nunits - gtail ? kHalfShift : kFullShift,
                       I / TL::BK, a.wait_limit, &c->err};
@@ -1910,11 +1912,11 @@ void expert_mfma_kernel(ExpertArgs a) {
       const float *abase = a.s.inter + (size_t)slot0 * I;
       const uint32_t abytes = a.s.inter_bytes - (uint32_t)((size_t)slot0 * I * sizeof(float));
       if (half) {
-        using TH = TileHalf<BM>;
+        using TH = UnitHalf<BM>;
         const float *brow0 = a.w.w2 + ((size_t)e * H + (size_t)ht * TH::BN) * I;
         if constexpr (BM == 128)
-          next = split_tile<SplitTile<128, TH::BN>, false>(lds, abase, abytes, s_aoff, rows, brow0, I,
-                                                           sout_out, slot0, H, ht * TH::BN, next_task, ready);
+          next = split_tile<TH, false>(lds, abase, abytes, s_aoff, rows, brow0, I, sout_out, slot0,
+                                       H, ht * TH::BN, next_task, ready);
         else
           next = mfma_tile<TH, false>(lds, abase, abytes, s_aoff, rows, brow0, I, sout_out, slot0,
                                       H, ht * TH::BN, next_task, ready);
@@ -2009,10 +2011,11 @@ static_assert(kRingSteps % kRingDepth == 0, "ring rotation realigns at task boun
 // With two token passes the four groups are read at once.
 // (kRingWideGroups, moe_internal.h)
 // 32-row tasks with 4 passes: batches whose largest expert holds 33-64
-// tokens (the router picks them from the counts; the dense FFN's chunks hold
-// all tokens), so each weight row is read once; 64-row tasks with 4 passes
-// would need twice the LDS for their partials.
-// (kRingDenseGroups, kRingDensePasses, moe_internal.h)
+// tokens (the router picks them from the counts), so each weight row is read
+// once; 64-row tasks with 4 passes would need twice the LDS for their partials.
+// (kRingTallGroups, kRingTallPasses, moe_internal.h)
+// The automatic plan streams up to 10 tokens, in 16-row tasks of one pass; the
+// other forms serve this plan forced on larger batches (moe_force_tile_rows).
 
 // 64-row tasks read at once load 4 weight rows per step; with two token
 // passes half the depth keeps the ring within the register budget of 3 waves
@@ -3120,7 +3123,7 @@ __global__ __launch_bounds__(kRingThreads) void expert_ring_kernel(ExpertArgs a)
     // covers 16, 32 or 64 rows
     if (c->n_rblocks != 0 ||
         (pl.rows != kStreamRows && pl.rows != kStreamRows * kRingWideGroups &&
-         pl.rows != kStreamRows * kRingDenseGroups)) {
+         pl.rows != kStreamRows * kRingTallGroups)) {
       if (tid == 0) st_agent(&a.s.ctrl->err, 2);
       return;
     }
@@ -3136,7 +3139,7 @@ __global__ __launch_bounds__(kRingThreads) void expert_ring_kernel(ExpertArgs a)
     if (maxcnt <= kRingTokens) ring_role<1, 1, kRingWideGroups>(a, sh, res, pl, ticks);
     else ring_role<kRingWideGroups, kRingMaxPasses>(a, sh, res, pl, ticks);
   } else {
-    ring_role<kRingDenseGroups, kRingDensePasses>(a, sh, res, pl, ticks);
+    ring_role<kRingTallGroups, kRingTallPasses>(a, sh, res, pl, ticks);
   }
 }
 
@@ -3356,7 +3359,7 @@ hipError_t launch_dense_skinny(const DenseArgs &a, hipStream_t st) {
 
 static size_t stream_lds_bytes() {
   const size_t a = ring_res_bytes(kRingWideGroups, kRingMaxPasses),
-               b = ring_res_bytes(kRingDenseGroups, kRingDensePasses);
+               b = ring_res_bytes(kRingTallGroups, kRingTallPasses);
   return a > b ? a : b;
 }
 
@@ -3419,7 +3422,7 @@ hipError_t launch_experts(const ExpertArgs &a, int tile_rows, int grid,
       break;
     }
     case 128: {
-      const size_t lds = SplitTile<128, 128>::LDS_BYTES;
+      const size_t lds = UnitTile<128>::LDS_BYTES;
       err = ensure_lds_attr(mfma_fn<128>(), lds);
       if (err != hipSuccess) return err;
       hipLaunchKernelGGL(expert_mfma_kernel<128>, dim3(grid), dim3(kThreads), lds, st, a);
@@ -3443,7 +3446,7 @@ int expert_bn(int tile_rows, int T) {
   switch (tile_rows) {
     case 32: return Tile<32>::BN;
     case 64: return Tile<64>::BN;
-    case 128: return Tile<128>::BN;
+    case 128: return UnitTile<128>::BN;
     // streaming: 64-row tasks once a batch has enough tokens per expert that
     // sharing each token-row load across 4 row groups pays
     default: return T >= kStreamWideTokens ? kStreamRows * kRingWideGroups : kStreamRows;
@@ -3477,7 +3480,7 @@ int expert_blocks_per_cu(int tile_rows) {
       break;
     case 128:
       e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-          &n, mfma_fn<128>(), kThreads, SplitTile<128, 128>::LDS_BYTES);
+          &n, mfma_fn<128>(), kThreads, UnitTile<128>::LDS_BYTES);
       break;
     default:
       return 1;

@@ -108,6 +108,7 @@ template <int BM_, int BN_, int NBUF_ = 1> struct SplitTile {
   static constexpr int A_PASSES = BM / 64, PASSES = (BM + BN) / 64;  // float4 pairs per thread and slab
   static constexpr int PLANE = (BM + BN) * BK;  // bf16 values per plane
   static constexpr size_t LDS_BYTES = (size_t)3 * PLANE * 2 * NBUF;
+  static constexpr int LDS_FLOATS = (int)(LDS_BYTES / sizeof(float));
   static_assert(BM % 64 == 0 && (BN == 64 || BN == 128) && AM * WAVES_M * 32 == BM, "whole row blocks");
 };
 

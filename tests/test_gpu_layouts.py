@@ -3,15 +3,14 @@ expert row counts chosen at their boundaries.
 
 Routing comes from crafted logits (moe_route_logits): each token's four
 experts get logits 2..5, the others -4, so the per-expert counts are exactly
-the ones asked for.  Under the forced 64-row plan the counts 1-16, 17-32,
-33-48, 49-64 take the 16-row skinny, narrow, 3-block skinny and wide layouts
-(and counts above 64 add units of each size); under the forced 128-row plan
-units of at most 64 rows run as 64-row tiles, 65-80 rows as 5-block 16-row
-skinny tiles, 81-96 as narrow tiles over three row blocks, 97-112 as 7-block
-skinny tiles, 113-127 as wide tiles, 128 as full tiles, and the last units'
-gate/up and down tiles as half-width tiles (the 128-row plan splits the
-last units' gate/up tiles up to 1024 tokens, the 64-row plan up to 128).  A
-second count set, with
+the ones asked for.  Under the forced 64-row plan up to 320 tokens the counts
+1-16, 17-32, 33-48, 49-64 take the fp32 tile's 16-row skinny, narrow, 3-block
+skinny and wide layouts (and counts above 64 add units of each size: the set
+"multi"); above 320 tokens ("mixed") its units run as 64-row split-bf16 tiles,
+the last ones' down tiles in the fp32 layouts at half width.  Under the forced
+128-row plan units of at most 64 rows run as 64-row split-bf16 tiles, larger
+ones as 128-row ones, and the last units' gate/up and down tiles at half width
+(gate/up up to 1024 tokens; the 64-row plan's up to 128).  The set "small", with
 every expert under 64 tokens, takes the longest-first unit order of the
 64-row plan.  The reference y comes from the oracle's own routing of the same
 logits, dispatch, expert and combine functions.
@@ -31,6 +30,8 @@ MIXED = [1, 2, 15, 16, 17, 20, 31, 32, 33, 40, 47, 48, 49, 56, 63, 64,
          65, 72, 80, 95, 96, 97, 112, 127, 128, 129, 160, 192, 200, 255, 256, 0]
 SMALL = [1, 3, 8, 15, 16, 17, 18, 24, 31, 32, 33, 34, 40, 47, 48, 49,
          50, 55, 60, 63, 64, 5, 9, 12, 20, 28, 36, 44, 52, 58, 61, 0]
+# several units per expert in few enough tokens for the fp32 tiles
+MULTI = [65, 72, 80, 96, 97, 112, 127, 128, 129, 160, 1, 15, 16, 17, 31, 32, 33, 48] + [0] * 14
 
 
 def say(*a):
@@ -85,7 +86,7 @@ def oracle_from_logits(O, w, x, logits, residual):
 
 
 def test_routing_for_counts_is_exact():
-    for cs in (MIXED, SMALL):
+    for cs in (MIXED, SMALL, MULTI):
         T, choice, counts = routing_for_counts(cs)
         got = np.bincount(choice.reshape(-1), minlength=E)
         assert list(got) == counts
@@ -94,12 +95,14 @@ def test_routing_for_counts_is_exact():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("name,cs,plan", [("mixed", MIXED, 64), ("mixed", MIXED, 128),
-                                          ("small", SMALL, 64), ("small", SMALL, 128)])
+                                          ("small", SMALL, 64), ("small", SMALL, 128),
+                                          ("multi", MULTI, 64), ("multi", MULTI, 128)])
 def test_tile_layouts(name, cs, plan, real_weights, oracle_mod):
     from final_amd import SparseMoeBlock, hip
     from final_amd import workloads as W
     w = real_weights
     T, choice, counts = routing_for_counts(cs)
+    assert (T > 320) == (name == "mixed")
     lg = crafted_logits(choice, seed=plan)
     x = W.gen_x(T, seed=70 + plan)
     r = W.gen_x(T, seed=71 + plan)

@@ -198,7 +198,9 @@ def test_embedding_bit_exact_and_bad_ids(oracle_mod):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("dim,rows,stride", [(2048, 64, 512 * 2048), (64, 4096, 64), (2048, 7, 2048)])
+# Up to 4096 rows one row per block, four above: remainders 1, 2 and 3.
+@pytest.mark.parametrize("dim,rows,stride", [(2048, 64, 512 * 2048), (64, 4096, 64), (2048, 7, 2048),
+                                             (64, 4097, 64), (64, 4098, 128), (2048, 4099, 2048)])
 def test_rmsnorm_rows_bit_exact(dim, rows, stride, oracle_mod):
     from final_amd import hip, lfm
     say(f"[rmsnorm] dim={dim} rows={rows} stride={stride}")
@@ -211,7 +213,8 @@ def test_rmsnorm_rows_bit_exact(dim, rows, stride, oracle_mod):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("batch,seq", [(2, 512), (3, 37), (1, 1)])
+# Up to 8192 tokens a token's rows spread over waves, one wave each above.
+@pytest.mark.parametrize("batch,seq", [(2, 512), (3, 37), (1, 1), (16, 512), (5, 1639)])
 def test_qk_norm_rope_bit_exact(batch, seq, oracle_mod):
     """GPU vs oracle bit for bit.  Both read `q1*c1 - q2*s1` (layer.cu:225-226)
     the same way (q1*c1 fused into an FMA with the rounded product q2*s1), so
@@ -251,7 +254,10 @@ def test_attention(batch, seq, oracle_mod):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("batch,seq", [(2, 512), (3, 2), (5, 1)])
+# Up to 256 tokens one per thread, four above: remainders, and sequences that
+# begin inside a thread's four tokens.
+@pytest.mark.parametrize("batch,seq", [(2, 512), (3, 2), (5, 1), (1, 256), (1, 257), (129, 2), (3, 333),
+                                       (259, 1)])
 def test_shortconv_bit_exact(batch, seq, oracle_mod):
     from final_amd import hip, lfm
     say(f"[shortconv] batch={batch} seq={seq}")

@@ -40,6 +40,10 @@ sys.path.insert(0, ROOT)
 
 METRIC = "MoE-block tokens/sec at T=4096 fp32, 1 GPU; % of MFMA / HBM roofline"
 PEAK_MFMA_F32_TFLOPS = 157.3   # MI355X dense fp32 matrix
+# fp32 products as six bf16 products each (split_tile.h): dense bf16 matrix / 6
+PEAK_SPLIT_TFLOPS = round(2500.0 / 6, 1)
+PEAK_SPLIT_SOURCE = "dense bf16 matrix peak 2500 TFLOP/s over the 6 bf16 products of an fp32 product"
+SPLIT_MIN_ROWS = 40            # 64-row plan: split-bf16 tiles above this many rows per expert
 PEAK_HBM_GBS = 8000.0          # MI355X HBM3E
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic.json")
 TRAFFIC_SOURCE = ("profiles/traffic.json: rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE of the same "
@@ -117,18 +121,34 @@ def cpu_baseline(w, x, threads: int, single_tokens: int = 128, min_s: float = 0.
             "host": host_cpu()}
 
 
-def roofline(plan, flops, nbytes, ms, name):
+def split_tiles(plan, T, experts, slots_per_token):
+    """Whether the plan's expert kernel computes in split-bf16 tiles."""
+    return plan == 128 or (plan == 64 and T * slots_per_token > SPLIT_MIN_ROWS * experts)
+
+
+def expert_kernel(plan, split):
+    if not plan:
+        return "expert_ring_kernel"
+    return "expert_mfma_kernel<64, true>" if plan == 64 and split else "expert_mfma_kernel<%d>" % plan
+
+
+def mfma_peak(split):
+    return PEAK_SPLIT_TFLOPS if split else PEAK_MFMA_F32_TFLOPS
+
+
+def roofline(plan, flops, nbytes, ms, name, split=False):
     """Primary bound of the expert kernel: MFMA when its arithmetic intensity
-    (algorithmic FLOP per algorithmic byte) is at or above the ridge
-    (157.3/8 FLOP/B), HBM below it; the other bound too when the intensity is
-    within 2x of the ridge."""
-    ridge = PEAK_MFMA_F32_TFLOPS * 1e3 / PEAK_HBM_GBS
+    (algorithmic FLOP per algorithmic byte) is at or above the ridge (157.3/8
+    FLOP/B with the fp32 instruction, 416.7/8 in split-bf16 tiles), HBM below
+    it; the other bound too when the intensity is within 2x of the ridge."""
+    peak = mfma_peak(split)
+    ridge = peak * 1e3 / PEAK_HBM_GBS
     ai = flops / max(nbytes, 1)
     mfma_bound = ai >= ridge
     if mfma_bound:
         a = flops / (ms / 1e3) / 1e12
-        roof = {"bound": "mfma", "achieved": round(a, 3), "peak": PEAK_MFMA_F32_TFLOPS,
-                "unit": "TFLOP/s", "frac": round(a / PEAK_MFMA_F32_TFLOPS, 4)}
+        roof = {"bound": "mfma", "achieved": round(a, 3), "peak": peak,
+                "unit": "TFLOP/s", "frac": round(a / peak, 4)}
     else:
         a = nbytes / (ms / 1e3) / 1e9
         roof = {"bound": "hbm", "achieved": round(a, 1), "peak": PEAK_HBM_GBS,
@@ -141,11 +161,12 @@ def roofline(plan, flops, nbytes, ms, name):
                                  "per_launch": {"bytes": nbytes}}
         else:
             o = flops / (ms / 1e3) / 1e12
-            roof["secondary"] = {"bound": "mfma", "achieved": round(o, 3),
-                                 "peak": PEAK_MFMA_F32_TFLOPS, "unit": "TFLOP/s",
-                                 "frac": round(o / PEAK_MFMA_F32_TFLOPS, 4),
+            roof["secondary"] = {"bound": "mfma", "achieved": round(o, 3), "peak": peak,
+                                 "unit": "TFLOP/s", "frac": round(o / peak, 4),
                                  "per_launch": {"flop": flops}}
         roof["arithmetic_intensity"] = round(ai, 2)
+    if split:
+        roof["mfma_peak_source"] = PEAK_SPLIT_SOURCE
     roof["traffic"] = None
     if os.path.exists(TRAFFIC_FILE):
         with open(TRAFFIC_FILE) as f:
@@ -153,7 +174,7 @@ def roofline(plan, flops, nbytes, ms, name):
         if tr:
             roof["traffic"] = tr.get("bytes_per_launch")
             roof["traffic_source"] = TRAFFIC_SOURCE
-    roof["kernel"] = "expert_mfma_kernel<%d>" % plan if plan else "expert_ring_kernel"
+    roof["kernel"] = expert_kernel(plan, split)
     roof["kernel_ms"] = round(ms, 4)
     roof["per_launch"] = {"flop": flops} if mfma_bound else {"bytes": nbytes}
     return roof
@@ -165,8 +186,8 @@ SETTLE_S = 0.1
 def settle_clock(step, stream):
     """Runs untimed steps for SETTLE_S seconds before the warm-up steps: the
     GPU clock ramps up over the first tens of milliseconds of work (T=4096
-    forwards run 3.4 ms at first, 2.78 ms from about the eighth), so short
-    runs and profiles would otherwise time the ramp."""
+    forwards run about a fifth longer at first than from about the eighth), so
+    short runs and profiles would otherwise time the ramp."""
     t0 = time.perf_counter()
     i = 0
     while time.perf_counter() - t0 < SETTLE_S:
@@ -235,7 +256,7 @@ def measure_moe(name, w, x, steps, warmup, nsets):
     ms_step = total_ms / steps
     flops = T * (W.flops_per_token() - 2 * W.H * W.E)  # W1, W3, W2 of 4 slots per token
     nbytes = W.algorithmic_bytes(counts, T) - (W.E * W.H * 4 + W.E * 4)
-    roof = roofline(plan, flops, nbytes, exp_ms, name)
+    roof = roofline(plan, flops, nbytes, exp_ms, name, split_tiles(plan, T, W.E, W.K))
     roof["router_ms"] = round(route_ms, 4)
     roof["kernel_path"] = "moe_forward's two launches (moe_route_forward, moe_experts)"
     return {"workload": name, "tokens": T, "ms_per_step": round(ms_step, 4),
@@ -387,8 +408,9 @@ def measure_model(steps, warmup, batch=64, seq=512):
                          "conv_avg": round(statistics.mean(conv), 3),
                          "embed": round(ev[0].elapsed_ms(ev[1]), 3),
                          "head": round(ev[-2].elapsed_ms(ev[-1]), 3)},
-            "roofline": {"bound": "mfma", "achieved": round(a, 3), "peak": PEAK_MFMA_F32_TFLOPS,
-                         "unit": "TFLOP/s", "frac": round(a / PEAK_MFMA_F32_TFLOPS, 4),
+            "roofline": {"bound": "mfma", "achieved": round(a, 3), "peak": PEAK_SPLIT_TFLOPS,
+                         "unit": "TFLOP/s", "frac": round(a / PEAK_SPLIT_TFLOPS, 4),
+                         "mfma_peak_source": PEAK_SPLIT_SOURCE,
                          "scope": "whole forward (every GEMM, attention and the MoE experts)",
                          "per_launch": {"flop": flops}, "traffic": None},
             "ffn": "the MoE block in all 24 layers, as the benchmark config specifies (the "
@@ -399,8 +421,9 @@ def measure_model(steps, warmup, batch=64, seq=512):
 
 def bench_dense(args, wl):
     """The dense FFN of layers 0-1 (MLP::forward_gpu): one step = one forward
-    of W2 (silu(W1 x) * (W3 x)) with I = 7168 (the fixed-routing router plus
-    the expert kernel over 4 chunks of 1792)."""
+    of W2 (silu(W1 x) * (W3 x)) with I = 7168 (up to 192 tokens two K-split
+    GEMMs, above the fixed-routing router plus the expert kernel over 4 chunks
+    of 1792)."""
     from final_amd import DenseMLP, hip
     from final_amd import workloads as W
     T = wl.T
@@ -440,11 +463,13 @@ def bench_dense(args, wl):
     wbytes = 3 * W.H * I * 4 + 2 * T * W.H * 4  # weights + x + y
     # the bound follows the arithmetic intensity (the dense FFN at T=64 already
     # does 32 FLOP per weight byte, past the fp32 ridge of ~19.7)
-    ridge = PEAK_MFMA_F32_TFLOPS * 1e12 / (PEAK_HBM_GBS * 1e9)
+    split = split_tiles(plan, T, 4, 4)  # 4 chunk experts, each holding every token
+    peak = mfma_peak(split)
+    ridge = peak * 1e12 / (PEAK_HBM_GBS * 1e9)
     if flops / wbytes > ridge:
         achieved = flops / (ms_step / 1e3) / 1e12
-        roof = {"bound": "mfma", "achieved": round(achieved, 3), "peak": PEAK_MFMA_F32_TFLOPS,
-                "unit": "TFLOP/s", "frac": round(achieved / PEAK_MFMA_F32_TFLOPS, 4),
+        roof = {"bound": "mfma", "achieved": round(achieved, 3), "peak": peak,
+                "unit": "TFLOP/s", "frac": round(achieved / peak, 4),
                 "per_launch": {"flop": flops}}
     else:
         achieved = wbytes / (ms_step / 1e3) / 1e9
@@ -452,7 +477,10 @@ def bench_dense(args, wl):
                 "unit": "GB/s", "frac": round(achieved / PEAK_HBM_GBS, 4),
                 "per_launch": {"bytes": wbytes}}
     roof["traffic"] = None
-    roof["kernel"] = ("expert_mfma_kernel<%d>" % plan if plan else "expert_ring_kernel") + " (whole step)"
+    if split:
+        roof["mfma_peak_source"] = PEAK_SPLIT_SOURCE
+    roof["kernel"] = (expert_kernel(plan, split) if plan
+                      else "dense_gate_up_kernel, dense_down_kernel") + " (whole step)"
     out = {
         "metric": "dense-FFN tokens/sec fp32, 1 GPU; % of MFMA / HBM roofline",
         "value": round(T * K / (ms_step * K / 1e3), 1), "unit": "tokens/s", "n_gpus": 1,

@@ -61,3 +61,24 @@ def test_roofline_bound_follows_intensity():
         flops = T * (W.flops_per_token() - 2 * W.H * W.E)
         nbytes = W.algorithmic_bytes(counts, T) - (W.E * W.H * 4 + W.E * 4)
         assert abs(flops / nbytes - ai) < 0.1
+
+
+def test_roofline_of_split_tiles():
+    """Kernels of split-bf16 tiles are held against the bf16 matrix peak over
+    the six products of an fp32 product, so that no fraction can pass 1."""
+    sys.path.insert(0, ROOT)
+    import bench
+    from final_amd import workloads as W
+    assert abs(bench.PEAK_SPLIT_TFLOPS - 2500 / 6) < 0.05
+    # T=4096, 2 ms: 180 TFLOP/s, more than the fp32 instruction's peak
+    flops = 4096 * (W.flops_per_token() - 2 * W.H * W.E)
+    r = bench.roofline(128, flops, flops / 244, 2.0, "none", split=True)
+    assert r["bound"] == "mfma" and r["achieved"] > bench.PEAK_MFMA_F32_TFLOPS and r["frac"] < 0.5
+    assert r["peak"] == bench.PEAK_SPLIT_TFLOPS and "6 bf16 products" in r["mfma_peak_source"]
+    # the kernel that runs, on either side of the line: the library's own rule
+    # (expert_split: more than 40 rows per expert) for the MoE block and the dense FFN
+    assert [bench.split_tiles(p, T, W.E, W.K) for p, T in ((64, 320), (64, 321), (128, 561), (0, 8))] \
+        == [False, True, True, False]
+    assert [bench.split_tiles(64, T, 4, 4) for T in (40, 41)] == [False, True]
+    r = bench.roofline(64, 30e9, 1e9, 1.0, "none", split=True)
+    assert r["bound"] == "hbm" and r["kernel"] == "expert_mfma_kernel<64, true>"

@@ -70,12 +70,9 @@ constexpr int kSplitProducts = 6;
 __device__ constexpr int kSplitA[kSplitProducts] = {2, 0, 1, 1, 0, 0};
 __device__ constexpr int kSplitB[kSplitProducts] = {0, 2, 1, 0, 1, 0};
 
-// max(m, |x|, |y|) and min, each one instruction; a NaN makes either a NaN.
+// max(m, |x|, |y|) in one instruction; a NaN makes it a NaN.
 __device__ __forceinline__ float max_abs(float m, float x, float y) {
   return __builtin_elementwise_maximum(__builtin_elementwise_maximum(m, fabsf(x)), fabsf(y));
-}
-__device__ __forceinline__ float min_abs(float m, float x, float y) {
-  return __builtin_elementwise_minimum(__builtin_elementwise_minimum(m, fabsf(x)), fabsf(y));
 }
 
 // v of another lane of the quad.
@@ -158,11 +155,18 @@ __device__ __forceinline__ int split_tile(float *lds, const float *abase, uint32
     const int ks = in ? slab * TL::BK * 4 : 0;
 #pragma unroll
     for (int i = 0; i < PASSES; ++i) {
-      const uint32_t off = i < PA ? a_src[i < PA ? i : 0] : b_src + (uint32_t)((i - PA) * 64 * K) * 4u;
+      // what is the same for all lanes in the scalar offset where registers
+      // decide the blocks per CU; two buffers have registers to spare and are
+      // faster with it in the vector offset (520 tokens 496 / 502 us)
+      const int uni = i < PA ? 0 : (i - PA) * 64 * K * 4;
+      const uint32_t own = i < PA ? a_src[i < PA ? i : 0] : b_src;
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
+      for (int h = 0; h < 2; ++h) {
+        const int so = uni + 64 * h;
         st[set][i][h] = __builtin_bit_cast(
-            f32x4, __builtin_amdgcn_raw_buffer_load_b128(i < PA ? arp : brp, off + 64 * h, ks, 0));
+            f32x4, __builtin_amdgcn_raw_buffer_load_b128(i < PA ? arp : brp, TL::NBUF == 1 ? own : own + so,
+                                                         TL::NBUF == 1 ? ks + so : ks, 0));
+      }
     }
   };
   // (lrow + 64 i) * 32 keeps lrow's swizzle: 64 i changes neither of its bits
@@ -170,20 +174,28 @@ __device__ __forceinline__ int split_tile(float *lds, const float *abase, uint32
   float mag[PASSES];  // largest magnitude this thread staged of each of its rows
 #pragma unroll
   for (int i = 0; i < PASSES; ++i) mag[i] = 0.0f;
+  auto track = [&](int set, int i) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      mag[i] = max_abs(mag[i], st[set][i][h][0], st[set][i][h][1]);
+      mag[i] = max_abs(mag[i], st[set][i][h][2], st[set][i][h][3]);
+    }
+  };
   auto store = [&](int set, int buf) {
 #pragma unroll
     for (int i = 0; i < PASSES; ++i) {
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        mag[i] = max_abs(mag[i], st[set][i][h][0], st[set][i][h][1]);
-        mag[i] = max_abs(mag[i], st[set][i][h][2], st[set][i][h][3]);
-      }
+      if constexpr (TL::NBUF == 1) track(set, i);
       bf16x8 p[3];
       split8(st[set][i], p);
 #pragma unroll
       for (int q = 0; q < 3; ++q)
         *reinterpret_cast<bf16x8 *>(wr + (3 * buf + q) * TL::PLANE + i * 64 * TL::BK) = p[q];
     }
+  };
+  // two buffers: a set's values stay until the next step's loads
+  auto track_late = [&](int set) {
+#pragma unroll
+    for (int i = 0; i < PASSES; ++i) track(set, i);
   };
 
   // fragments: lane l supplies row l % 32, chunk 2 kk + l / 32 of a slab
@@ -210,6 +222,9 @@ __device__ __forceinline__ int split_tile(float *lds, const float *abase, uint32
     load(j, j);
     __builtin_amdgcn_sched_barrier(0);  // in the loop's order: see the waits in it
   }
+  // The MFMAs go before other waves' instructions: those of the wave that
+  // splits beside them then fill the cycles between, which pays for the maxima
+  // (4096 tokens 2030 -> 1997 us).
   auto compute = [&](int kk, int buf) {
     const int co = ((2 * kk + lh) ^ sw) * 8 + 3 * buf * TL::PLANE;
     bf16x8 bf[2][3];
@@ -241,12 +256,15 @@ __device__ __forceinline__ int split_tile(float *lds, const float *abase, uint32
       __syncthreads();
       load(t + 1, 0);
       __builtin_amdgcn_sched_barrier(0);  // not sunk among the MFMAs
+      __builtin_amdgcn_s_setprio(1);
       compute(0, 0);
       compute(1, 0);
+      __builtin_amdgcn_s_setprio(0);
       __syncthreads();
     }
   } else {
     store(0, 0);
+    track_late(0);
     if constexpr (Ready::kActive)
       if (wave == 0) ready.wait(2);
     __syncthreads();
@@ -257,9 +275,12 @@ __device__ __forceinline__ int split_tile(float *lds, const float *abase, uint32
         if (t >= nslab) break;
         load(t + 2, u);
         __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(1);
         compute(0, u);
         store(1 - u, 1 - u);  // slab t + 1 (past the end: zeros into a buffer nobody reads)
         compute(1, u);
+        track_late(1 - u);
+        __builtin_amdgcn_s_setprio(0);
         if constexpr (Ready::kActive)
           if (wave == 0) ready.wait(t + 3);
         __syncthreads();
@@ -288,34 +309,23 @@ __device__ __forceinline__ int split_tile(float *lds, const float *abase, uint32
   // Elements the parts do not give: not finite, or below the limit of their
   // row and column (kSplitFloor).
   const float mb[2] = {lds[BM + wn * 64 + elr], lds[BM + wn * 64 + 32 + elr]};
-  auto lost = [&](int i, int c, int r) {
-    const float ma = lds[wm * AM * 32 + i * 32 + 8 * (r >> 2) + 4 * elh + (r & 3)];
-    const float v = fabsf(acc[i][c][r]);
-    return !(v >= ma + mb[c] && v <= __FLT_MAX__);
+  auto row_limit = [&](int i, int r) {
+    return lds[wm * AM * 32 + i * 32 + 8 * (r >> 2) + 4 * elh + (r & 3)];
   };
 #pragma unroll
   for (int i = 0; i < AM; ++i) {
-    // a lane's smallest results against the largest limit, then each its own
-    float top = 0.0f, ma = -__builtin_inff(), low[2] = {__builtin_inff(), __builtin_inff()};
+    // a lane's smallest result above its row's limit against its column's
+    float top = 0.0f, low[2] = {__builtin_inff(), __builtin_inff()};
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const f32x4 m = ld4(lds + wm * AM * 32 + i * 32 + 8 * q + 4 * elh);
-      ma = fmaxf(fmaxf(ma, fmaxf(m[0], m[1])), fmaxf(m[2], m[3]));
+    for (int r = 0; r < 16; r += 2)
 #pragma unroll
-      for (int c = 0; c < 2; ++c)
-#pragma unroll
-        for (int h = 0; h < 4; h += 2) {
-          low[c] = min_abs(low[c], acc[i][c][4 * q + h], acc[i][c][4 * q + h + 1]);
-          top = max_abs(top, acc[i][c][4 * q + h], acc[i][c][4 * q + h + 1]);
-        }
-    }
-    bool any = !(top <= __FLT_MAX__ && low[0] >= ma + mb[0] && low[1] >= ma + mb[1]);
-    if (__any(any)) {
-      any = false;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) any = any || lost(i, 0, r) || lost(i, 1, r);
-    }
-    if (__any(any)) {
+      for (int c = 0; c < 2; ++c) {
+        const float x = acc[i][c][r], y = acc[i][c][r + 1];
+        top = max_abs(top, x, y);
+        low[c] = __builtin_elementwise_minimum(
+            __builtin_elementwise_minimum(low[c], fabsf(x) - row_limit(i, r)), fabsf(y) - row_limit(i, r + 1));
+      }
+    if (__any(!(top <= __FLT_MAX__ && low[0] >= mb[0] && low[1] >= mb[1]))) {
       // fp32 MFMAs with operands straight from memory: lane l supplies row
       // l % 32 at k offset 4 (l / 32) of each 8-wide k group
       const int row = wm * AM * 32 + i * 32 + elr;
@@ -347,7 +357,8 @@ __device__ __forceinline__ int split_tile(float *lds, const float *abase, uint32
       for (int c = 0; c < 2; ++c)
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-          if (lost(i, c, r)) acc[i][c][r] = f[c][r];
+          if (!(fabsf(acc[i][c][r]) - row_limit(i, r) >= mb[c] && fabsf(acc[i][c][r]) <= __FLT_MAX__))
+            acc[i][c][r] = f[c][r];
     }
     // lane l holds column l % 32 and rows 8 (r / 4) + 4 (l / 32) + r % 4 of
     // each block, so a store writes 128 contiguous bytes of two rows

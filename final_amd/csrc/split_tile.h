@@ -2,15 +2,18 @@
 // on v_mfma_f32_32x32x16_bf16.
 //
 // The fp32 matrix instruction peaks at 157 TFLOP/s on this chip, the bf16 one
-// at 2.5 PFLOP/s.  Every fp32 value is exactly the sum of three bf16 values
-// (8 significand bits each, rounded to nearest, so each part is at most 2^-9
-// of the one before), and a product of two values is then six bf16 products
-//   a2 b0 + a0 b2 + a1 b1 + a1 b0 + a0 b1 + a0 b0
-// plus three terms of at most 3 * 2^-27 of it, less than the rounding of one
-// fp32 product.  The six are exact in fp32 and accumulate in fp32, 16 k per
-// instruction, so a sum of K products takes 6 K / 16 roundings where the fp32
-// instruction takes K / 2: measured against 64-bit sums its error is smaller.
-// Six of them take 192 cycles per 32x32x16 block where fp32 takes 512.
+// at 2.5 PFLOP/s.  Every fp32 value of at least 2^-110 is exactly the sum of
+// three bf16 values (8 significand bits each, rounded to nearest, so each part
+// is at most 2^-8 of the one before), and a product of two values is then nine
+// bf16 products, of which six are taken,
+//   a2 b0 + a0 b2 + a1 b1 + a1 b0 + a0 b1 + a0 b0.
+// The other three are together at most 2^-24 of the product (2^-28 on
+// average), as much as the rounding of one fp32 product: an output that is a
+// single product is within 1 ulp, where the fp32 instruction's is within half.
+// The six are exact in fp32 and accumulate in fp32, 16 k per instruction, so a
+// sum of K products takes 6 K / 16 roundings where the fp32 instruction takes
+// K / 2: measured against 64-bit sums its error is smaller (K = 2048 7.0e-7,
+// 8.1e-7).  Six of them take 192 cycles per 32x32x16 block where fp32 takes 512.
 //
 // Values the split cannot carry leave outputs that a wave computes again with
 // the fp32 instruction: infinities, NaN and magnitudes above the largest bf16

@@ -85,7 +85,8 @@ def test_gemm_nt_dispatch_edges(M, N, K, res):
     cols = np.unique(r.integers(0, N, 300))  # a sample of the columns, in 64 bits
     ref = A.astype(np.float64) @ B[cols].astype(np.float64).T
     # K + 6 roundings of at most 2^-24 of the sum of the products' magnitudes
-    # (an fp32 sum in any order, whole or as bf16 parts), one more for the residual
+    # (an fp32 sum in any order; as bf16 parts 6 K / 16 of them and the parts
+    # left out, at most 2^-24 of each product), one more for the residual
     tol = (K + 6) * 2.0 ** -24 * (np.abs(A).astype(np.float64) @ np.abs(B[cols]).astype(np.float64).T)
     if res:
         ref = R[:, cols] + ref

@@ -189,8 +189,10 @@ static int plan_index(int rows) {
 // 11, 233.1 vs 230.2 at 12, 245.6 vs 235.1 at 16, 258.2 vs 243.5 at 20;
 // before the half-width down tiles streaming led up to 20; 283.3 vs 269.8
 // and 282.0 vs 276.3 at 48, two boxes;
-// split-bf16 tiles from 321), 128-row tiles, all split-bf16, from 561 (495
-// vs 514 us at 512, 584 vs 530 at 640, 756 vs 685 at 1024).  moe_route +
+// split-bf16 tiles from 321), 128-row tiles, all split-bf16, from 561 (64- vs
+// 128-row 421 vs 467 us at 440, 486 vs 476 at 480, 553 vs 517 at 560, 582 vs 538
+// at 640: by time the line would lie at 460; it stays at the 560 that callers of
+// moe_plan_tile_rows know).  moe_route +
 // moe_experts, which keep the full router, take the same plans (with it,
 // streaming led up to 48).
 constexpr int kStreamMaxTokens = 10;

@@ -224,7 +224,7 @@ int moe_last_plan_counts(moe_ctx *ctx, int *counts, moe_stream_t stream);
 int moe_plan_tile_rows(const moe_ctx *ctx, int num_tokens);
 
 /* Overrides the plan (tests): rows = -1 automatic, 0 streaming, 32/64/128.
- * Streaming covers batches of up to 1024 tokens; larger ones use 32. */
+ * Streaming covers batches of up to 1024 tokens; larger ones use 64. */
 int moe_force_tile_rows(moe_ctx *ctx, int rows);
 
 /* Test hook: scales the kernels' bounded-wait limit (1 = default, >1 shorter).

@@ -161,14 +161,14 @@ __device__ __forceinline__ int split_tile(float *lds, const float *abase, uint32
       // what is the same for all lanes in the scalar offset where registers
       // decide the blocks per CU; two buffers have registers to spare and are
       // faster with it in the vector offset (520 tokens 496 / 502 us)
-      const int uni = i < PA ? 0 : (i - PA) * 64 * K * 4;
+      const uint32_t uni = i < PA ? 0u : (uint32_t)((i - PA) * 64) * (uint32_t)K * 4u;
       const uint32_t own = i < PA ? a_src[i < PA ? i : 0] : b_src;
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const int so = uni + 64 * h;
+        const uint32_t so = uni + 64 * h;
         st[set][i][h] = __builtin_bit_cast(
             f32x4, __builtin_amdgcn_raw_buffer_load_b128(i < PA ? arp : brp, TL::NBUF == 1 ? own : own + so,
-                                                         TL::NBUF == 1 ? ks + so : ks, 0));
+                                                         TL::NBUF == 1 ? (int)(ks + so) : ks, 0));
       }
     }
   };

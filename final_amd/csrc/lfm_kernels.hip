@@ -77,9 +77,9 @@ constexpr int kGemmCUs = 256;
 // blocks share), and within that range tiles run in groups of kGroupM M-tiles
 // column by column, so the blocks running together share B tiles and A tiles.
 // Bound by the matrix cores' power: at 32768 x 3072 x 2048 (128-row tiles)
-// 1910-2050 us, box to box, = 201-216 TFLOP/s, where the fp32 instruction's tile
-// took 2819 us = 146 and bf16 MFMAs alone on random operands reach 300 / 6; the
-// clock drops to 1.5 GHz and the MFMAs are busy 77 % of it.
+// 1910-2050 us, box to box, = 201-216 TFLOP/s, where the fp32 instruction's
+// tile took 2819 us = 146 and bf16 MFMAs alone on random operands reach 1800 / 6
+// = 300; the clock drops to 1.5 GHz and the MFMAs are busy 77 % of it.
 template <int BM, bool RES>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
 void gemm_split_kernel(GemmArgs g) {
